@@ -56,10 +56,15 @@ constexpr int kSizeBuckets = 64;
 // partials (one workgroup per request and kv-head) stays short.
 constexpr int kMaxSmallItems = 16;
 
-// One 1024-thread workgroup builds the plan.
+// One 1024-thread workgroup builds the plan.  Latency bound: a chain of small
+// reads, scans and barriers, so what counts is how many there are (8 requests
+// of up to 512 tokens 10.2 us -> 6.4 us, one request of 8192 11.3 -> 7.3 us by
+// the parallel size search and bucket scan below and by keeping a window's
+// counts in registers).
 __device__ inline void decode_plan_body(const PlanParams& p) {
   __shared__ int smem[16];
   __shared__ int s_bucket[kSizeBuckets];
+  __shared__ int s_pages[1024];
   int total_pages = 0;
   if (p.num_pages) {
     for (int base = 0; base < p.batch; base += 1024) {
@@ -91,18 +96,25 @@ __device__ inline void decode_plan_body(const PlanParams& p) {
     // Page counts are read once (batch <= 1024: one request per thread).
     const bool one = p.batch <= 1024;
     int mine = 0;  // pages of this thread's request if this kernel serves it
-    if (one && (int)threadIdx.x < p.batch) {
-      int np = 0;
-      if (count_of((int)threadIdx.x, 1, np) > 0) mine = np;
-    }
-    auto items_at = [&](int c) {  // the workgroup's item count at c pages per item
-      if (one) return block_sum_1024(mine > 0 ? (mine + c - 1) / c : 0, smem);
-      int cnt = 0;
-      for (int base = 0; base < p.batch; base += 1024) {
-        const int b = base + (int)threadIdx.x;
+    if (one) {
+      if ((int)threadIdx.x < p.batch) {
         int np = 0;
-        cnt += block_sum_1024(b < p.batch ? count_of(b, c, np) : 0, smem);
+        if (count_of((int)threadIdx.x, 1, np) > 0) mine = np;
       }
+      s_pages[threadIdx.x] = mine;
+    }
+    auto items_at = [&](int c) {  // this wavefront's item count at c pages per item
+      int cnt = 0;
+      for (int b = (int)threadIdx.x & 63; b < p.batch; b += 64) {
+        if (one) {
+          cnt += (s_pages[b] + c - 1) / c;
+        } else {
+          int np = 0;
+          cnt += count_of(b, c, np);
+        }
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o, 64);
       return cnt;
     };
     int longest = 0;
@@ -123,19 +135,30 @@ __device__ inline void decode_plan_body(const PlanParams& p) {
     if (lo > hi) lo = hi;
     if (lo < 1) lo = 1;
     // The smallest size in [lo, hi] whose items fit the slots (counts fall as
-    // the size grows), or hi when none does.  Uniform across the workgroup:
-    // every thread sees the same totals.
-    if (lo < hi && items_at(hi) <= p.slots) {
-      int h = hi;
-      while (lo < h) {
-        const int mid = (lo + h) >> 1;
-        if (items_at(mid) <= p.slots) h = mid;
-        else lo = mid + 1;
+    // the size grows), or hi when none does.  Each round prices 16 sizes from
+    // lo to hi, one per wavefront, and keeps the gap below the first that fits:
+    // two rounds for the usual 16..64 pages (a binary search with the whole
+    // workgroup summing each size took seven, each with two barriers).
+    // Uniform across the workgroup: every thread sees the same counts.
+    const int w = (int)threadIdx.x >> 6, top = hi;
+    bool fits = true;
+    for (int l = lo, h = hi; l < h;) {
+      const int cnt = items_at(l + (h - l) * w / 15);
+      if ((threadIdx.x & 63) == 0) smem[w] = cnt;
+      __syncthreads();
+      const uint64_t ok = __builtin_amdgcn_ballot_w64(smem[threadIdx.x & 15] <= p.slots) & 0xffffu;
+      __syncthreads();
+      if (!ok) {
+        fits = false;
+        break;
       }
-      cp = lo;
-    } else {
-      cp = lo < hi ? hi : lo;
+      const int k = __builtin_ctzll(ok);  // the smallest size priced that fits
+      const int at = l + (h - l) * k / 15;
+      l = k == 0 ? at : l + (h - l) * (k - 1) / 15 + 1;
+      h = at;
+      lo = l;
     }
+    cp = fits ? lo : top;
   }
   if (threadIdx.x < kSizeBuckets) s_bucket[threadIdx.x] = 0;
   __syncthreads();
@@ -147,9 +170,11 @@ __device__ inline void decode_plan_body(const PlanParams& p) {
   };
   // pass 1: item offsets per request, full items in place, remainder histogram
   int carry = 0, carry_full = 0;
+  int np = 0, n = 0, full = 0, rb = -1;  // the thread's request (of the last window)
   for (int base = 0; base < p.batch; base += 1024) {
     const int b = base + (int)threadIdx.x;
-    int np = 0, n = 0, full = 0, rb = -1;
+    n = full = 0;
+    rb = -1;
     if (b < p.batch) items_of(b, np, n, full, rb);
     int total, total_full;
     const int first = block_exclusive_scan_1024(n, total, smem) + carry;
@@ -172,22 +197,26 @@ __device__ inline void decode_plan_body(const PlanParams& p) {
     carry_full += total_full;
   }
   __syncthreads();
-  // bucket start positions, largest bucket first, after all full items
-  if (threadIdx.x == 0) {
-    int off = carry_full;
-    for (int k = kSizeBuckets - 1; k >= 0; --k) {
-      const int c = s_bucket[k];
-      s_bucket[k] = off;
-      off += c;
+  // bucket start positions, largest bucket first, after all full items: an
+  // exclusive scan by one wavefront, lane k holding bucket 63 - k (one thread
+  // walking the buckets took 64 dependent LDS round trips, 4 us of the plan)
+  static_assert(kSizeBuckets == kWave, "one bucket per lane");
+  if (threadIdx.x < kSizeBuckets) {
+    const int k = kSizeBuckets - 1 - (int)threadIdx.x, c = s_bucket[k];
+    int x = c;
+#pragma unroll
+    for (int o = 1; o < kSizeBuckets; o <<= 1) {
+      const int y = __shfl_up(x, o, 64);
+      if ((int)threadIdx.x >= o) x += y;
     }
+    s_bucket[k] = carry_full + x - c;
   }
   __syncthreads();
   // pass 2: remainder items
   for (int base = 0; base < p.batch; base += 1024) {
     const int b = base + (int)threadIdx.x;
     if (b < p.batch) {
-      int np, n, full, rb;
-      items_of(b, np, n, full, rb);
+      if (p.batch > 1024) items_of(b, np, n, full, rb);  // one window: still in registers
       if (rb >= 0) {
         const int pos = atomicAdd(&s_bucket[rb], 1);
         if (pos < p.max_chunks) p.work[pos] = make_int4(b, full, np, n);
