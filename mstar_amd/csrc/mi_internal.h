@@ -116,29 +116,45 @@ int decode_run_impl(const void* q, int32_t q_dtype, int64_t q_stride_token, int6
                     int64_t out_stride_token, int64_t out_stride_head, int phases, hipStream_t stream,
                     bool ragged_pair = false);
 
+// Wavefront scans and reductions on the VALU's cross-lane paths: one row_shr
+// per power of two within a 16-lane row, then two row broadcasts.  (__shfl
+// goes through the LDS crossbar with address arithmetic around it; a plan
+// workgroup runs four wavefronts per SIMD, so every instruction of its scans
+// costs 16 cycles.)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_move(int old, int x) {
+  return __builtin_amdgcn_update_dpp(old, x, CTRL, ROWS, 0xf, false);
+}
+__device__ __forceinline__ int wave_inclusive_sum(int x) {
+  x += dpp_move<0x111, 0xf>(0, x);  // row_shr:1, 2, 4, 8
+  x += dpp_move<0x112, 0xf>(0, x);
+  x += dpp_move<0x114, 0xf>(0, x);
+  x += dpp_move<0x118, 0xf>(0, x);
+  x += dpp_move<0x142, 0xa>(0, x);  // row_bcast:15 into rows 1 and 3
+  x += dpp_move<0x143, 0xc>(0, x);  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+__device__ __forceinline__ int wave_sum(int x) { return __builtin_amdgcn_readlane(wave_inclusive_sum(x), 63); }
+__device__ __forceinline__ int wave_max(int x) {
+  constexpr int kMin = -0x7fffffff - 1;
+  x = max(x, dpp_move<0x111, 0xf>(kMin, x));
+  x = max(x, dpp_move<0x112, 0xf>(kMin, x));
+  x = max(x, dpp_move<0x114, 0xf>(kMin, x));
+  x = max(x, dpp_move<0x118, 0xf>(kMin, x));
+  x = max(x, dpp_move<0x142, 0xa>(kMin, x));
+  x = max(x, dpp_move<0x143, 0xc>(kMin, x));
+  return __builtin_amdgcn_readlane(x, 63);
+}
+
 // Exclusive prefix sum over a 1024-thread block; `smem` holds >= 16 ints.
 __device__ __forceinline__ int block_exclusive_scan_1024(int v, int& total, int* smem) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  int x = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int x = wave_inclusive_sum(v);
   if (lane == 63) smem[w] = x;
   __syncthreads();
-  if (w == 0) {
-    int t = lane < 16 ? smem[lane] : 0;
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) {
-      const int y = __shfl_up(t, o, 64);
-      if (lane >= o) t += y;
-    }
-    if (lane < 16) smem[lane] = t;
-  }
-  __syncthreads();
-  const int before = w ? smem[w - 1] : 0;
-  total = smem[15];
+  const int t = wave_inclusive_sum(lane < 16 ? smem[lane] : 0);  // every wavefront scans the 16 sums
+  total = __builtin_amdgcn_readlane(t, 15);
+  const int before = w ? __builtin_amdgcn_readlane(t, w - 1) : 0;
   __syncthreads();
   return before + x - v;
 }
@@ -147,26 +163,20 @@ __device__ __forceinline__ int block_exclusive_scan_1024(int v, int& total, int*
 // (smem: 16 ints, free again on return).
 __device__ __forceinline__ int block_sum_1024(int v, int* smem) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  v = wave_sum(v);
   if (lane == 0) smem[w] = v;
   __syncthreads();
-  int t = 0;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) t += smem[i];
+  const int t = wave_sum(lane < 16 ? smem[lane] : 0);
   __syncthreads();
   return t;
 }
 
 __device__ __forceinline__ int block_max_1024(int v, int* smem) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+  v = wave_max(v);
   if (lane == 0) smem[w] = v;
   __syncthreads();
-  int t = smem[0];
-#pragma unroll
-  for (int i = 1; i < 16; ++i) t = max(t, smem[i]);
+  const int t = wave_max(smem[lane & 15]);
   __syncthreads();
   return t;
 }

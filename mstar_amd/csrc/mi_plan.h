@@ -58,9 +58,9 @@ constexpr int kMaxSmallItems = 16;
 
 // One 1024-thread workgroup builds the plan.  Latency bound: a chain of small
 // reads, scans and barriers, so what counts is how many there are (8 requests
-// of up to 512 tokens 10.2 us -> 6.4 us, one request of 8192 11.3 -> 7.3 us by
-// the parallel size search and bucket scan below and by keeping a window's
-// counts in registers).
+// of up to 512 tokens took 10.2 us, 6.4 with the parallel size search and
+// bucket scan below and a window's counts kept in registers, 5.1 with scans that
+// stay off the LDS crossbar).
 __device__ inline void decode_plan_body(const PlanParams& p) {
   __shared__ int smem[16];
   __shared__ int s_bucket[kSizeBuckets];
@@ -113,9 +113,7 @@ __device__ inline void decode_plan_body(const PlanParams& p) {
           cnt += count_of(b, c, np);
         }
       }
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o, 64);
-      return cnt;
+      return wave_sum(cnt);
     };
     int longest = 0;
     if (one) {
@@ -203,13 +201,7 @@ __device__ inline void decode_plan_body(const PlanParams& p) {
   static_assert(kSizeBuckets == kWave, "one bucket per lane");
   if (threadIdx.x < kSizeBuckets) {
     const int k = kSizeBuckets - 1 - (int)threadIdx.x, c = s_bucket[k];
-    int x = c;
-#pragma unroll
-    for (int o = 1; o < kSizeBuckets; o <<= 1) {
-      const int y = __shfl_up(x, o, 64);
-      if ((int)threadIdx.x >= o) x += y;
-    }
-    s_bucket[k] = carry_full + x - c;
+    s_bucket[k] = carry_full + wave_inclusive_sum(c) - c;
   }
   __syncthreads();
   // pass 2: remainder items
