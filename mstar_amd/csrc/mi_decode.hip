@@ -48,20 +48,6 @@ constexpr int kMinChunkTokens = 1024;  // never split a request finer than this 
 // resident workgroups (decode_plan_body)
 constexpr int kSmallChunkTokens = 256;
 
-// Compute units of the current device (cached per device).
-static int device_cu_count() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!cached[dev]) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cached[dev] = n;
-  }
-  return cached[dev];
-}
-
-
 // Target number of wavefronts for one plan: ~4K (item, kv-head, quarter)
 // wave units fill 256 CUs x 2 resident workgroups about twice; with the
 // longest-first work order the drain tail stays short while few requests

@@ -5,6 +5,19 @@
 
 namespace mi {
 
+// Compute units of the current device (cached per device).
+inline int device_cu_count() {
+  static int cached[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (!cached[dev]) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cached[dev] = n;
+  }
+  return cached[dev];
+}
+
 // Workspace layout of a split-KV plan (decode kernel + merge).
 struct SplitLayout {
   int64_t hdr, chunk_indptr, work, lse, opart, total;

@@ -4,12 +4,13 @@
 //
 // plan:  one launch (prefill_plan_kernel): the token map (the per-new-token
 //        (page, slot) of flashinfer_utils.py:211-256), the tiles of every
-//        long-query request, costed and cut as (kv-head, tile) units into 8
-//        cost-balanced per-XCD queues, and, for the short-query requests
+//        long-query request, costed and put as (kv-head, tile) units, or
+//        pieces of them, into 8 per-XCD queues (pf_choose), and, for the short-query requests
 //        (qo_len * group <= 16, e.g. the decode rows of a mixed batch), a
 //        split-KV plan for the decode kernel in the same workspace.
 // run:   mi_prefill_short (decode kernel + merge for the short-query
-//        requests) and mi_prefill_tiles (prefill_kernel).
+//        requests) and mi_prefill_tiles (prefill_kernel, and the merge of
+//        tiles that the plan has cut into key pieces).
 //
 // prefill_kernel (persistent, one workgroup per CU): a unit is a tile of
 // 256 (query token, q-head) rows of one request and kv-head -- GQA rows
@@ -38,13 +39,44 @@ namespace mi {
 constexpr int kShortRows = kShortRowsMax;  // qo_len * group <= 16 -> decode kernel (8 on a paired plan)
 
 // Workspace: header | per-XCD queue counters + finished-workgroup counter |
-// tile list | tile cost prefix | unit order | decode split plan.
-// Header words: [0] tiles, [1] units (tiles x kv-heads), [8 + x] first unit
-// of XCD x's queue (x = 0..8, [16] = units).
+// tile list | tile cost prefix | unit order | decode split plan | (where room
+// is left) piece list | split tile list | piece partials (lse, o).
+// Header words: [kPfTiles] tiles, [kPfUnits] units (tiles x kv-heads, or
+// pieces x kv-heads when tiles are split), [kPfPieces] pieces per kv-head (0:
+// no tile is split), [kPfSplitTiles] split tiles, [kPfCuts + x] first unit of
+// XCD x's queue (x = 0..8, [16] = units).
 struct PrefillLayout {
   int64_t hdr, ctr, tiles, tcum, order, split;
   int32_t max_tiles;
 };
+
+// What a split of tiles into key pieces needs, behind the decode split plan:
+// as many partials as fit the workspace, up to kPfMaxParts (three rounds of
+// one piece per CU; a split of more pieces never paid).  parts == 0: no room.
+constexpr int32_t kPfMaxParts = 768;
+struct PfSplitLayout {
+  int64_t pieces, split_tiles, lse, o, total;
+  int32_t max_pieces, parts;
+};
+
+static PfSplitLayout pf_split_layout(int64_t base, int32_t max_tiles, int32_t nkv, int32_t head_dim, int64_t ws_avail) {
+  PfSplitLayout P{};
+  P.total = base;
+  const int64_t rows = pf_rows(head_dim);
+  const int64_t per_part = 16 + 16 + 4 * rows + 4 * rows * head_dim;
+  const int64_t fixed = 16LL * max_tiles + 5 * 256;
+  int64_t parts = kPfMaxParts;
+  if (ws_avail >= 0 && (ws_avail - base - fixed) / per_part < parts) parts = (ws_avail - base - fixed) / per_part;
+  if (parts < 2 * nkv) return P;
+  P.parts = (int32_t)parts;
+  P.max_pieces = max_tiles + P.parts;
+  P.pieces = mi_align_up(base, 256);
+  P.split_tiles = mi_align_up(P.pieces + 16LL * P.max_pieces, 256);
+  P.lse = mi_align_up(P.split_tiles + 16LL * P.parts, 256);
+  P.o = mi_align_up(P.lse + 4 * rows * P.parts, 256);
+  P.total = mi_align_up(P.o + 4 * rows * head_dim * P.parts, 256);
+  return P;
+}
 
 static PrefillLayout prefill_layout(int32_t batch, int32_t max_qo_tokens, int32_t group, int32_t nkv,
                                     int32_t head_dim) {
@@ -61,6 +93,14 @@ static PrefillLayout prefill_layout(int32_t batch, int32_t max_qo_tokens, int32_
   L.order = mi_align_up(L.tcum + 4LL * (L.max_tiles + 1), 256);
   L.split = mi_align_up(L.order + 4LL * L.max_tiles * nkv, 256);
   return L;
+}
+
+// The split layout of a plan or run call (shapes only, so the two agree).
+static PfSplitLayout pf_split_of(const PrefillLayout& L, int32_t batch, int32_t group, int32_t nkv, int32_t head_dim,
+                                 int64_t ws_bytes) {
+  const bool pair = pair_heads(nullptr, batch, nkv, group, head_dim, true);
+  const int64_t split = split_layout(batch, nkv, head_dim, ws_bytes < 0 ? -1 : ws_bytes - L.split, pair).total;
+  return pf_split_layout(L.split + split, L.max_tiles, nkv, head_dim, ws_bytes);
 }
 
 // ------------------------------------------------------------ token map
@@ -135,7 +175,196 @@ struct PfPlanArgs {
   int32_t* tcum;
   int32_t* order;
   int32_t* ctr;
+  // splitting tiles into key pieces (max_parts 0: never)
+  int32_t max_parts, workgroups;
+  float unit_steps, part_steps, merge_steps, merge_part_steps;  // costs in key steps (pf_split_costs)
+  int4* pieces;
+  int4* split_tiles;
 };
+
+// What a unit costs beyond its key steps, in key steps of the kernel.
+struct PfSplitCosts {
+  float unit, part, merge, merge_part;
+};
+static PfSplitCosts pf_split_costs(int head_dim) {
+  if (head_dim > 128) return {6.f, 3.f, 5.f, 0.03f};
+  return {7.f, 5.5f, 5.5f, 0.03f};
+}
+
+// How a plan's tiles go to the queues: as units in head-major order cut into
+// 8 runs of equal cost (kPfLocal: each XCD's L2 serves few K/V streams), or
+// dealt to the queues heaviest first (kPfWhole), or cut into key pieces of at
+// most `cap` steps and those dealt.
+//
+// A call with few tiles leaves most CUs idle unless they are cut (one
+// 512-token chunk at 32 q / 4 kv heads is 64 units for 256 CUs: 109 us of
+// prefill kernel uncut, 44 + 8 us of merge cut in four), and with two or three
+// units per CU a queue of one request's long units ends long after the others
+// (4 chunks of 512-2048 tokens, 32 q / 4 kv heads, fp8 cache: 437 us from the
+// local queues, 320 us dealt).  Where the local queues are as even as a deal
+// they stay: 8 x 2048 tokens at head_dim 256 1262 us local, 1286 us dealt.  Each candidate is priced, one wavefront each, by the bounds that
+// any schedule of units u_1 >= u_2 >= ... on m workgroups obeys: their mean
+// load, and (k + 1) u_{km + 1} for each k (of the km + 1 longest, k + 1 share
+// a workgroup).  Heaviest-first queues come close to the larger of the two.
+// The bounds are taken over all workgroups, and for kPfLocal also over each
+// queue's units on the queue's eighth of them.
+constexpr int kPfLocal = 0, kPfWhole = 0x7fffffff;
+constexpr int kPfCandidates = 8;
+__device__ inline int pf_candidate_cap(int i, float share) {
+  // in mean loads of a workgroup, and at least so many steps
+  constexpr float kShare[kPfCandidates] = {0.f, 2.4f, 1.7f, 1.35f, 1.15f, 1.f, .75f, .5f};
+  constexpr int kMin[kPfCandidates] = {0, 16, 8, 6, 4, 4, 4, 4};
+  return i == 0 ? kPfWhole : max(kMin[i], (int)ceilf(share * kShare[i]));
+}
+// prefix(t): cost of the tiles before tile t (one kv-head).  One histogram of
+// the units' costs per queue of kPfLocal serves all candidates, so the price
+// of a plan hardly grows with its tiles.
+template <typename Prefix>
+__device__ inline int pf_choose(const PfPlanArgs& a, int n_tiles, int64_t ct, int mc, Prefix prefix, int* s_bin) {
+  __shared__ float s_est[16];
+  constexpr int kBins = 128, kPer = kBins / 64;
+  const int tid = (int)threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int64_t total = ct * a.nkv, units = (int64_t)n_tiles * a.nkv;
+  const float share = (float)total / a.workgroups;
+  if (total == 0 || (units > 16LL * a.workgroups && mc < 0.1f * share)) return kPfLocal;  // many short units balance by themselves
+  // bin i: costs up to top(i), exact below 128 steps
+  const float width = mc < kBins ? 1.f : (float)(mc + 1) / kBins, inv_width = 1.f / width;
+  auto top = [&](int i) { return mc < kBins ? (float)i : (i + 1) * width; };
+  auto bin_of = [&](float c) { return min(kBins - 1, (int)(c * inv_width)); };
+  for (int i = tid; i < 16 * kBins; i += 1024) s_bin[i] = 0;
+  __syncthreads();
+  const float per_queue = 8.f / (float)total, ctf = (float)ct;
+  for (int h = 0; h < a.nkv; ++h)
+    for (int t = tid; t < n_tiles; t += 1024) {
+      const int p = prefix(t);
+      const int x = min(7, (int)((h * ctf + p) * per_queue));
+      atomicAdd(&s_bin[x * kBins + bin_of((float)(prefix(t + 1) - p))], 1);
+    }
+  __syncthreads();
+  // wavefronts 0..7: queue w of kPfLocal; 8..15: the dealt candidates
+  const bool local = w < 8;
+  const int cap = local ? kPfWhole : pf_candidate_cap(w - 8, share);
+  const float m = local ? max(1, a.workgroups / 8) : a.workgroups, inv_m = 1.f / m;
+  int* hist = s_bin + w * kBins;  // of the pieces
+  // (a bin's top is at least its units' costs: the piece counts are upper bounds)
+  const int biggest = cap == kPfWhole ? 1 : (mc + cap - 1) / cap;
+  int parts = 0;
+  if (!local) {
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int b = 64 * k + lane;
+      int cnt = 0;
+#pragma unroll
+      for (int x = 0; x < 8; ++x) cnt += s_bin[x * kBins + b];
+      if (cnt > 0) {
+        const int c = (int)ceilf(top(b));
+        const int n = cap == kPfWhole ? 1 : max(1, (c + cap - 1) / cap);
+        parts += n > 1 ? n * cnt : 0;
+        atomicAdd(&hist[bin_of((float)((c + n - 1) / n))], n * cnt);
+      }
+    }
+    parts = wave_sum(parts);
+  }
+  // lane l owns kPer bins from the top: ranks of its pieces by an exclusive scan
+  int cnt[kPer], mine = 0;
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) mine += cnt[k] = hist[kBins - 1 - kPer * lane - k];
+  const int upto = wave_inclusive_sum(mine), pieces = __builtin_amdgcn_readlane(upto, 63);
+  const float extra = a.unit_steps + (parts > 0 ? a.part_steps : 0.f);
+  float est = (share * m + pieces * a.unit_steps + parts * a.part_steps) * inv_m;
+  int rank = upto - mine;
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const float q = floorf((rank + cnt[k] - 0.5f) * inv_m);  // the last k with a (km + 1)-th longest piece in this bin
+    if (cnt[k] > 0 && q * m >= rank) est = fmaxf(est, (q + 1.f) * (top(kBins - 1 - kPer * lane - k) + extra));
+    rank += cnt[k];
+  }
+  est = bitcast<float>((uint32_t)wave_max(bitcast<int>(est)));  // non-negative floats order as ints
+  if (parts > 0) est += a.merge_steps + a.merge_part_steps * parts;
+  if (parts > a.max_parts || biggest > kPfMaxPieces || (cap != kPfWhole && parts == 0)) est = __builtin_inff();
+  if (lane == 0) s_est[w] = est;
+  __syncthreads();
+  float e_local = 0.f;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) e_local = fmaxf(e_local, s_est[k]);
+  // dealing gives up some L2 locality and a cut needs a merge: each has to win by a margin
+  int best = -1;
+  float e_best = 0.97f * e_local;
+#pragma unroll
+  for (int k = 0; k < kPfCandidates; ++k)
+    if (s_est[8 + k] < (best == 0 ? 0.97f : 1.f) * e_best) {
+      best = k;
+      e_best = s_est[8 + k];
+    }
+  return best < 0 ? kPfLocal : pf_candidate_cap(best, share);
+}
+
+// Lists the pieces of a cut and deals them to the queues.  Tile t's
+// n = ceil(cost / cap) pieces share its key steps evenly; split tiles get n
+// slots per kv-head and a merge entry.  The pieces of one kv-head are listed
+// heaviest first (a counting sort), and entry i of queue x is a closed form of
+// (i, x) (pf_dealt), so the queues themselves need no list.
+// mine: the thread's tile, where there is one tile per thread.
+template <typename Prefix>
+__device__ inline void pf_deal(const PfPlanArgs& a, int n_tiles, int cap, int mc, Prefix prefix, bool one, int2 mine,
+                               int* s_bin, int* smem) {
+  const int tid = (int)threadIdx.x;
+  auto pieces_of = [&](int c) { return cap == kPfWhole ? 1 : max(1, (c + cap - 1) / cap); };
+  const int most = min(cap, mc);
+  const float scale = most < 1024 ? 1.f : 1024.f / (float)(most + 1);
+  auto key_of = [&](int steps) { return 1023 - min(1023, (int)(steps * scale)); };
+  s_bin[tid] = 0;
+  __syncthreads();
+  // piece k of n covers steps [k c / n, (k + 1) c / n): c % n of them are one
+  // step longer than c / n
+  for (int t = tid; t < n_tiles; t += 1024) {
+    const int c = prefix(t + 1) - prefix(t), n = pieces_of(c), q = n == 1 ? c : c / n, r = c - q * n;
+    atomicAdd(&s_bin[key_of(q)], n - r);
+    if (r > 0) atomicAdd(&s_bin[key_of(q + 1)], r);
+  }
+  __syncthreads();
+  int np;
+  const int first = block_exclusive_scan_1024(s_bin[tid], np, smem);
+  s_bin[tid] = first;
+  int carry_slots = 0, carry_split = 0;
+  for (int t0 = 0; t0 < n_tiles; t0 += 1024) {
+    const int t = t0 + tid;
+    int n = 0, c = 0;
+    if (t < n_tiles) {
+      c = prefix(t + 1) - prefix(t);
+      n = pieces_of(c);
+    }
+    // slots (at most kPfMaxParts) and split tiles in one scan
+    int tot = 0;
+    const int at = cap == kPfWhole ? 0 : block_exclusive_scan_1024(n > 1 ? n << 16 | 1 : 0, tot, smem);
+    const int slot = a.nkv * (carry_slots + (at >> 16));
+    if (cap == kPfWhole) __syncthreads();  // s_bin is complete
+    if (t < n_tiles) {
+      const int2 te = one ? mine : a.tiles[t];
+      const int q = n == 1 ? c : c / n, r = c - q * n;
+      int at_short = atomicAdd(&s_bin[key_of(q)], n - r), at_long = r > 0 ? atomicAdd(&s_bin[key_of(q + 1)], r) : 0;
+      for (int k = 0, part = 0; k < n; ++k) {
+        part += r;
+        const bool longer = part >= n;
+        if (longer) part -= n;
+        a.pieces[longer ? at_long++ : at_short++] = make_int4(te.x, te.y, k | n << 16, slot);
+      }
+      if (n > 1) a.split_tiles[carry_split + (at & 0xffff)] = make_int4(te.x, te.y, n, slot);
+    }
+    carry_slots += tot >> 16;
+    carry_split += tot & 0xffff;
+  }
+  if (tid < 64) {
+    const int len = tid < 8 ? pf_dealt_len(np, a.nkv, tid) : 0;
+    const int at = wave_inclusive_sum(len) - len;
+    if (tid < 9) a.hdr[kPfCuts + tid] = at;
+  }
+  if (tid == 0) {
+    a.hdr[kPfUnits] = np * a.nkv;
+    a.hdr[kPfPieces] = np;
+    a.hdr[kPfSplitTiles] = carry_split;
+  }
+}
 
 // One 1024-thread workgroup.  Requests go in windows of 1024 (one per
 // thread: tile count, exclusive scan); the window's tiles are then listed
@@ -148,9 +377,11 @@ __device__ inline void prefill_plan_body(const PfPlanArgs& a) {
   __shared__ int s_first[1025];  // window-relative first tile of each request, [1024] = window total
   __shared__ int s_kvl[1024], s_qol[1024];
   __shared__ int s_bin[8 * 1024];
+  __shared__ int s_cum[1025];  // cost prefix of the first 1024 tiles
   const int tid = (int)threadIdx.x;
   const int group = a.group, tile_rows = a.tile_rows, causal = a.causal, max_tiles = a.max_tiles;
-  int carry = 0, carry_cost = 0;
+  int carry = 0, carry_cost = 0, mc = 0;
+  int2 mine = make_int2(0, 0);  // the thread's last tile
   for (int base = 0; base < a.batch; base += 1024) {
     const int b = base + tid;
     int n = 0;
@@ -183,61 +414,82 @@ __device__ inline void prefill_plan_body(const PfPlanArgs& a) {
       int tot_cost;
       const int cum = block_exclusive_scan_1024(cost, tot_cost, smem);
       if (j < total && carry + j < max_tiles) {
-        a.tiles[carry + j] = make_int2(base + r, row0);
+        mine = make_int2(base + r, row0);
+        a.tiles[carry + j] = mine;
         a.tcum[carry + j] = carry_cost + cum;
+        if (carry + j < 1024) s_cum[carry + j] = carry_cost + cum;
+        mc = max(mc, cost);
       }
       carry_cost += tot_cost;
     }
     carry += total;
     __syncthreads();  // s_first / s_kvl / s_qol are rewritten by the next window
   }
-  const int n_tiles = min(carry, max_tiles);
-  if (tid == 0) a.tcum[n_tiles] = carry_cost;  // truncated lists keep a consistent prefix end
+  const int listed = min(carry, max_tiles);
+  if (tid == 0) {
+    a.tcum[listed] = carry_cost;  // truncated lists keep a consistent prefix end
+    if (listed <= 1024) s_cum[listed] = carry_cost;
+  }
   __threadfence_block();
   __syncthreads();
   const int64_t ct = carry_cost;
-  const int64_t units = (int64_t)n_tiles * a.nkv;
   const int64_t total = ct * a.nkv;
+  const int n_tiles = listed;
+  if (tid < 9) a.ctr[tid * kCtrStride] = 0;  // queues of the first run
   if (tid == 0) {
-    a.hdr[0] = n_tiles;
-    a.hdr[1] = (int32_t)units;
+    a.hdr[kPfTiles] = n_tiles;
+    a.hdr[kPfPieces] = 0;
+    a.hdr[kPfSplitTiles] = 0;
   }
-  // Queue cuts: queue x starts at the first unit whose cost prefix
-  // h*ct + tcum[t] (unit u = h*n_tiles + t) reaches ceil(x * total / 8).
-  // The prefix never decreases, so that unit is the one u with
-  // prefix(u-1) < target <= prefix(u); every thread tests its units.
-  if (tid <= 8) s_cut[tid] = tid == 0 ? 0 : (int)units;
-  __syncthreads();
-  if (total > 0) {
-    auto prefix = [&](int64_t u) -> int64_t {
-      const int64_t h = u / n_tiles, t = u - h * n_tiles;
-      return h * ct + a.tcum[t];
-    };
-    for (int64_t u = 1 + tid; u < units; u += 1024) {
-      const int64_t pu = prefix(u), pp = prefix(u - 1);
-#pragma unroll
-      for (int x = 1; x < 8; ++x) {
-        const int64_t target = (x * total + 7) / 8;
-        if (pp < target && target <= pu) s_cut[x] = (int)u;
-      }
+  const int32_t* tcum = a.tcum;
+  auto prefix = [&](int t) { return n_tiles <= 1024 ? s_cum[t] : tcum[t]; };
+  if (a.max_parts > 0) {
+    mc = block_max_1024(mc, smem);
+    const int cap = pf_choose(a, n_tiles, ct, mc, prefix, s_bin);
+    if (cap != kPfLocal) {
+      pf_deal(a, n_tiles, cap, mc, prefix, a.batch <= 1024 && n_tiles <= 1024, mine, s_bin, smem);
+      return;
     }
   }
+  const int units = n_tiles * a.nkv;
+  if (tid == 0) a.hdr[kPfUnits] = units;
+  // Queue cuts: queue x starts at the first unit whose cost prefix
+  // h*ct + prefix(t) (unit u = h*n_tiles + t) reaches ceil(x * total / 8).
+  // The prefix never decreases, so that unit is the one u with
+  // prefix(u-1) < target <= prefix(u); every thread tests its units.
+  if (tid <= 8) s_cut[tid] = tid == 0 ? 0 : units;
   __syncthreads();
-  if (tid <= 8) a.hdr[8 + tid] = s_cut[tid];
+  if (total > 0) {
+    for (int h = 0; h < a.nkv; ++h)
+      for (int t = tid; t < n_tiles; t += 1024) {
+        if (h + t == 0) continue;
+        const int64_t pu = h * ct + prefix(t), pp = t > 0 ? h * ct + prefix(t - 1) : (h - 1) * ct + prefix(n_tiles - 1);
+#pragma unroll
+        for (int x = 1; x < 8; ++x) {
+          const int64_t target = (x * total + 7) >> 3;
+          if (pp < target && target <= pu) s_cut[x] = h * n_tiles + t;
+        }
+      }
+  }
+  __syncthreads();
+  if (tid <= 8) a.hdr[kPfCuts + tid] = s_cut[tid];
   // Within each queue, units go heaviest first: one counting sort over
   // (queue, 1023 - min(cost, 1023)) keys in LDS.  Queues are contiguous unit
   // ranges, so the sorted positions of queue x start at its first unit.
   for (int i = tid; i < 8 * 1024; i += 1024) s_bin[i] = 0;
+  int cut[8];
+#pragma unroll
+  for (int k = 1; k < 8; ++k) cut[k] = uniform(s_cut[k]);
   __syncthreads();
-  const int32_t* tcum = a.tcum;
-  auto key_of = [&](int u) {
+  auto key_of = [&](int h, int t) {
+    const int u = h * n_tiles + t;
     int x = 0;
 #pragma unroll
-    for (int k = 1; k < 8; ++k) x += u >= s_cut[k];
-    const int t = u % n_tiles;
-    return x * 1024 + 1023 - min(tcum[t + 1] - tcum[t], 1023);
+    for (int k = 1; k < 8; ++k) x += u >= cut[k];
+    return x * 1024 + 1023 - min(prefix(t + 1) - prefix(t), 1023);
   };
-  for (int u = tid; u < (int)units; u += 1024) atomicAdd(&s_bin[key_of(u)], 1);
+  for (int h = 0; h < a.nkv; ++h)
+    for (int t = tid; t < n_tiles; t += 1024) atomicAdd(&s_bin[key_of(h, t)], 1);
   __syncthreads();
   {
     int loc[8], sum = 0;  // thread t owns bins [8t, 8t + 8)
@@ -248,13 +500,12 @@ __device__ inline void prefill_plan_body(const PfPlanArgs& a) {
     }
     int tot;
     const int base = block_exclusive_scan_1024(sum, tot, smem);
-    __syncthreads();
 #pragma unroll
     for (int k = 0; k < 8; ++k) s_bin[8 * tid + k] = base + loc[k];
   }
   __syncthreads();
-  for (int u = tid; u < (int)units; u += 1024) a.order[atomicAdd(&s_bin[key_of(u)], 1)] = u;
-  if (tid < 9) a.ctr[tid * kCtrStride] = 0;  // queues of the first run
+  for (int h = 0; h < a.nkv; ++h)
+    for (int t = tid; t < n_tiles; t += 1024) a.order[atomicAdd(&s_bin[key_of(h, t)], 1)] = h * n_tiles + t;
 }
 
 // The whole plan in one launch: workgroup 0 lists and orders the MFMA tiles,
@@ -282,6 +533,94 @@ static int launch_prefill(const PrefillParams& pp, int head_dim, int grid, hipSt
   return MI_OK;
 }
 
+// Merge of split tiles, after the prefill kernel.  A wavefront merges NV output
+// tiles of one (split tile, kv-head, row group): row r is
+// sum_i 2^(lse_i - max) o_i / sum_i 2^(lse_i - max), in piece order, up to 8
+// pieces (4 at head_dim 256) loaded together.  HBM/latency bound: 64 tiles cut
+// in four (33 MB of partials) 8 us.  (Merged by the
+// prefill kernel's own workgroups once all pieces were done, the partials
+// crossing the XCDs' L2 caches by agent-scope stores or by fences, the same 64
+// tiles took 63 and 84 us of kernel against 44 + 8.)
+constexpr int kPfMergeThreads = 512;
+template <typename MT, int D>
+__global__ __launch_bounds__(kPfMergeThreads) void prefill_merge_kernel(PrefillParams p) {
+  constexpr int VW = D / 16, NV = D / 64, ROWS = pf_rows(D), NG = ROWS / 16, U = D > 128 ? 4 : 8, WAVES = kPfMergeThreads / 64;
+  constexpr float kNegInf = -__builtin_inff();
+  const int nkv = p.num_kv_heads, G = p.group;
+  const int lane = lane_id(), col = lane & 15, grp = lane >> 4;
+  const int total = p.hdr[kPfSplitTiles] * nkv * NG * 4;
+  for (int w = uniform((int)blockIdx.x * WAVES + ((int)threadIdx.x >> 6)); w < total; w += (int)gridDim.x * WAVES) {
+    const int part = w & 3, rgi = (w >> 2) % NG, th = (w >> 2) / NG;
+    const int h = th % nkv;
+    const int4 st = p.split_tiles[th / nkv];
+    const int b = uniform(st.x), n = uniform(st.z), slot = uniform(st.w) + h * n;
+    const int qo_start = p.qo_indptr[b];
+    const int rows_total = (p.qo_indptr[b + 1] - qo_start) * G;
+    const int row = uniform(st.y) + 16 * rgi + col;
+    if (row >= rows_total) continue;
+    float4 acc[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    float M = kNegInf, wsum = 0.f;
+    for (int c = 0; c < n; c += U) {
+      float lse[U];
+      float4 o[U][NV];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        lse[u] = kNegInf;
+        if (c + u < n) {
+          const int64_t s = slot + c + u;
+          lse[u] = p.part_lse[s * ROWS + 16 * rgi + col];
+          const float4* src = p.part_o + ((s * NG + rgi) * VW + NV * part) * 64 + lane;
+#pragma unroll
+          for (int i = 0; i < NV; ++i) o[u][i] = src[64 * i];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (lse[u] == kNegInf) continue;  // past the last piece, or one that this row sees no key of
+        if (lse[u] > M) {
+          const float sc = fast_exp2(M - lse[u]);
+          wsum *= sc;
+#pragma unroll
+          for (int i = 0; i < NV; ++i) {
+            acc[i].x *= sc;
+            acc[i].y *= sc;
+            acc[i].z *= sc;
+            acc[i].w *= sc;
+          }
+          M = lse[u];
+        }
+        const float g = fast_exp2(lse[u] - M);  // a NaN lse makes the row NaN
+        wsum += g;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+          acc[i].x += g * o[u][i].x;
+          acc[i].y += g * o[u][i].y;
+          acc[i].z += g * o[u][i].z;
+          acc[i].w += g * o[u][i].w;
+        }
+      }
+    }
+    const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
+    const int tok = row / G, g = row - tok * G;
+    uint16_t* orow = (uint16_t*)p.out + (int64_t)(qo_start + tok) * p.out_stride_tok + (int64_t)(h * G + g) * p.out_stride_head;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      *(uint2*)(orow + 16 * (NV * part + i) + 4 * grp) =
+          make_uint2(MT::pack2(acc[i].x * inv, acc[i].y * inv), MT::pack2(acc[i].z * inv, acc[i].w * inv));
+  }
+}
+
+template <typename MT>
+static void launch_prefill_merge(const PrefillParams& pp, int head_dim, int grid, hipStream_t stream) {
+  switch (head_dim) {
+    case 64: hipLaunchKernelGGL((prefill_merge_kernel<MT, 64>), dim3(grid), dim3(kPfMergeThreads), 0, stream, pp); break;
+    case 128: hipLaunchKernelGGL((prefill_merge_kernel<MT, 128>), dim3(grid), dim3(kPfMergeThreads), 0, stream, pp); break;
+    default: hipLaunchKernelGGL((prefill_merge_kernel<MT, 256>), dim3(grid), dim3(kPfMergeThreads), 0, stream, pp); break;
+  }
+}
+
 static bool ok_head_dim(int d) { return d == 64 || d == 128 || d == 256; }
 
 }  // namespace mi
@@ -292,7 +631,7 @@ extern "C" int64_t mi_prefill_workspace_bytes(int32_t batch, int32_t max_qo_toke
   if (batch < 0 || max_qo_tokens < 0 || num_kv_heads <= 0 || num_qo_heads <= 0 || num_qo_heads % num_kv_heads)
     return MI_ERR_INVALID;
   const PrefillLayout L = prefill_layout(batch, max_qo_tokens, num_qo_heads / num_kv_heads, num_kv_heads, head_dim);
-  return L.split + split_layout(batch, num_kv_heads, head_dim, -1).total;
+  return pf_split_of(L, batch, num_qo_heads / num_kv_heads, num_kv_heads, head_dim, -1).total;
 }
 
 extern "C" int32_t mi_prefill_short_rows(int32_t batch, int32_t num_qo_heads, int32_t num_kv_heads,
@@ -342,6 +681,16 @@ extern "C" int mi_prefill_plan(const int32_t* qo_indptr, const int32_t* kv_indpt
   a.tcum = (int32_t*)(ws + L.tcum);
   a.order = (int32_t*)(ws + L.order);
   a.ctr = (int32_t*)(ws + L.ctr);
+  const PfSplitLayout P = pf_split_of(L, batch, G, num_kv_heads, head_dim, workspace_bytes);
+  const PfSplitCosts costs = pf_split_costs(head_dim);
+  a.max_parts = P.parts;
+  a.workgroups = device_cu_count();
+  a.unit_steps = costs.unit;
+  a.part_steps = costs.part;
+  a.merge_steps = costs.merge;
+  a.merge_part_steps = costs.merge_part;
+  a.pieces = (int4*)(ws + P.pieces);
+  a.split_tiles = (int4*)(ws + P.split_tiles);
   TokenMapArgs m;
   m.qo_indptr = qo_indptr;
   m.kv_indptr = kv_indptr;
@@ -451,6 +800,11 @@ static int prefill_run_impl(const void* q, int32_t q_dtype, int64_t q_stride_tok
   pp.tiles = (const int2*)(ws + L.tiles);
   pp.order = (const int32_t*)(ws + L.order);
   pp.ctr = (int32_t*)((uint8_t*)workspace + L.ctr);
+  const PfSplitLayout P = pf_split_of(L, batch, G, nkv, D, workspace_bytes);
+  pp.pieces = (const int4*)(ws + P.pieces);
+  pp.split_tiles = (const int4*)(ws + P.split_tiles);
+  pp.part_lse = (float*)((uint8_t*)workspace + P.lse);
+  pp.part_o = (float4*)((uint8_t*)workspace + P.o);
   pp.out = out;
   pp.out_stride_tok = out_stride_token;
   pp.out_stride_head = out_stride_head;
@@ -459,18 +813,24 @@ static int prefill_run_impl(const void* q, int32_t q_dtype, int64_t q_stride_tok
   pp.page_size = kv->page_size;
   pp.causal = causal ? 1 : 0;
   pp.scale_log2 = sm_scale * 1.4426950408889634f;
-  // persistent grid: one workgroup per CU (each holds two wavefronts per SIMD),
-  // never more than there are units
-  int dev = 0, ncu = 256;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return MI_ERR_LAUNCH;
-  const int64_t units = (int64_t)L.max_tiles * nkv;
+  // persistent grid: one workgroup per CU (each holds two wavefronts per
+  // SIMD), never more than there can be units
+  const int ncu = device_cu_count();
+  const int64_t units = (int64_t)(P.parts > 0 ? P.max_pieces : L.max_tiles) * nkv;
   const int grid = (int)(((units < ncu ? units : (int64_t)ncu) + 7) / 8 * 8);
   if (q_dtype == MI_BF16)
     st = fp8 ? launch_prefill<BF16, true>(pp, D, grid, s) : launch_prefill<BF16, false>(pp, D, grid, s);
   else
     st = fp8 ? launch_prefill<F16, true>(pp, D, grid, s) : launch_prefill<F16, false>(pp, D, grid, s);
   if (st != MI_OK) return st;
+  // which tiles are split is the device's decision: the merge is launched
+  // wherever a split is possible, and exits at once without one (4 us)
+  if (P.parts > 0) {
+    const int64_t waves = (int64_t)L.max_tiles * nkv * (pf_rows(D) / 16) * 4, per = kPfMergeThreads / 64;
+    const int mgrid = (int)(waves < ncu * per ? (waves + per - 1) / per : ncu);
+    if (q_dtype == MI_BF16) launch_prefill_merge<BF16>(pp, D, mgrid, s);
+    else launch_prefill_merge<F16>(pp, D, mgrid, s);
+  }
   MI_CHECK_LAUNCH();
   return MI_OK;
 }

@@ -22,6 +22,9 @@ constexpr int pf_rows(int head_dim) { return 16 * pf_rg(head_dim) * pf_waves(hea
 constexpr int kPfKeys = 32;                // keys per K/V tile
 constexpr int kPfTileCap = 1024;           // tiles whose row-group addresses are staged in LDS at a time
 constexpr int kCtrStride = 32;  // one 128-byte line per XCD counter
+// Header words of the prefill plan (see mi_prefill.hip).
+enum { kPfTiles = 0, kPfUnits, kPfPieces, kPfSplitTiles, kPfCuts = 8 };
+constexpr int kPfMaxPieces = 1024;  // key pieces of one tile (their index and count share an int)
 
 // ------------------------------------------------------------ attention
 struct PrefillParams {
@@ -39,11 +42,123 @@ struct PrefillParams {
   const int2* tiles;
   const int32_t* order;
   int32_t* ctr;
+  // Dealt plans (hdr[kPfPieces] != 0): units are (kv-head, piece) instead of
+  // (kv-head, tile), and a queue's entries follow from their place (pf_dealt).
+  const int4* pieces;        // (request, first row, piece index | pieces of the tile << 16, the tile's first slot)
+  const int4* split_tiles;   // (request, first row, pieces, first slot)
+  float4* part_o;            // [slot][row group of 16][D/16][64 lanes], normalised
+  float* part_lse;           // [slot][tile rows]
   void* out;
   int64_t out_stride_tok, out_stride_head;
   int32_t num_kv_heads, group, page_size, causal;
   float scale_log2;
 };
+
+// A unit's tile and, for a piece of a split tile, which part of the tile's
+// key steps it covers and where its partial goes.
+struct PfUnit {
+  int h, b, row0, k, n, slot;  // slot: the piece's own partial (n > 1)
+};
+
+// Dealt plans: np pieces per kv-head, heaviest first, dealt to the 8 queues so
+// that each XCD sees as few heads as an even deal allows: 8 / nkv XCDs per
+// head, or nkv / 8 heads per XCD; other head counts deal (piece, head) pairs
+// in turn.  Entries of queue x, and the piece and head of entry i.
+__host__ __device__ inline int pf_dealt_len(int np, int nkv, int x) {
+  if (nkv <= 8 && 8 % nkv == 0) {
+    const int r = 8 / nkv;
+    return (np - x % r + r - 1) / r;
+  }
+  if (nkv % 8 == 0) return np * (nkv / 8);
+  return (np * nkv - x + 7) / 8;
+}
+__host__ __device__ inline void pf_dealt(int nkv, int x, int i, int& piece, int& h) {
+  if (nkv <= 8 && 8 % nkv == 0) {
+    const int r = 8 / nkv;
+    h = x / r;
+    piece = i * r + x % r;
+  } else if (nkv % 8 == 0) {
+    const int r = nkv / 8;
+    piece = i / r;
+    h = x + 8 * (i - piece * r);
+  } else {
+    piece = (8 * i + x) / nkv;
+    h = 8 * i + x - piece * nkv;
+  }
+}
+
+// The next unit of this workgroup as (queue | place in it << 3), -1 when all
+// queues are empty.  Called by one wavefront; lanes 0..7 look at the 8 queues
+// at once (starting with the XCD's own), so a claim costs its own round trips
+// and not one per queue passed: read one after the other, the empty queues
+// took a workgroup 1-2 us each when it ran out of work.
+MI_DEVICE int pf_claim(const PrefillParams& p) {
+  const int lane = lane_id();
+  const int y = ((int)blockIdx.x + lane) & 7;  // workgroups are dispatched to the 8 XCDs round-robin
+  const int len = p.hdr[kPfCuts + 1 + y] - p.hdr[kPfCuts + y];
+  int i = 0x7fffffff;
+  if (lane == 0) i = __hip_atomic_fetch_add(p.ctr + y * kCtrStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  int u = uniform(i < len ? i << 3 | y : -1);
+  if (u >= 0) return u;
+  const int taken = __hip_atomic_load(p.ctr + y * kCtrStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  uint64_t left = __builtin_amdgcn_ballot_w64(lane > 0 && lane < 8 && taken < len);
+  while (left) {
+    const int src = __builtin_ctzll(left);
+    left &= left - 1;
+    i = 0x7fffffff;
+    if (lane == src) i = __hip_atomic_fetch_add(p.ctr + y * kCtrStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    u = __builtin_amdgcn_readlane(i < len ? i << 3 | y : -1, src);
+    if (u >= 0) return u;
+  }
+  return -1;
+}
+
+MI_DEVICE PfUnit pf_unit(const PrefillParams& p, int claim) {
+  PfUnit r;
+  const int x = claim & 7, i = claim >> 3;
+  if (p.hdr[kPfPieces] == 0) {
+    const int nt = p.hdr[kPfTiles];
+    const int unit = p.order[p.hdr[kPfCuts + x] + i];
+    r.h = unit / nt;
+    const int2 te = p.tiles[unit - r.h * nt];
+    r.b = te.x;
+    r.row0 = te.y;
+    r.k = 0;
+    r.n = 1;
+    r.slot = 0;
+  } else {
+    int piece;
+    pf_dealt(p.num_kv_heads, x, i, piece, r.h);
+    const int4 pe = p.pieces[piece];
+    r.b = pe.x;
+    r.row0 = pe.y;
+    r.k = pe.z & 0xffff;
+    r.n = pe.z >> 16;
+    r.slot = pe.w + r.h * r.n + r.k;
+  }
+  return r;
+}
+
+// One row group's partial: VW output tiles in the MFMA layout, and each row's
+// log-sum-exp (-inf: the row sees no key of the piece; NaN: it met a NaN or
+// +inf score).
+template <int VW, int ROWS>
+MI_DEVICE void pf_put_part(const PrefillParams& p, int slot, int rgi, const f32x4 (&o)[VW], float inv, float lse) {
+  float4* po = p.part_o + ((int64_t)slot * (ROWS / 16) + rgi) * VW * 64 + lane_id();
+#pragma unroll
+  for (int jj = 0; jj < VW; ++jj) po[64 * jj] = make_float4(o[jj][0] * inv, o[jj][1] * inv, o[jj][2] * inv, o[jj][3] * inv);
+  if (lane_id() < 16) p.part_lse[(int64_t)slot * ROWS + 16 * rgi + lane_id()] = lse;
+}
+// The last workgroup to finish resets the queues for the next run with this
+// plan.  Every claim of the others has returned by then (each workgroup adds
+// itself after its last claim), so no fence is needed.
+MI_DEVICE void pf_done(const PrefillParams& p) {
+  if (threadIdx.x == 0 && __hip_atomic_fetch_add(p.ctr + 8 * kCtrStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                              (int)gridDim.x - 1) {
+#pragma unroll
+    for (int y = 0; y < 9; ++y) __hip_atomic_store(p.ctr + y * kCtrStride, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
 
 template <typename MT, bool FP8, int D>
 struct PrefillCfg {
@@ -78,32 +193,21 @@ __global__ __launch_bounds__(64 * pf_waves(D)) void prefill_kernel(PrefillParams
   // byte offset (from the head's base) of the first row of each 16-row group of the staged tiles
   __shared__ int64_t lds_toff[2 * kPfTileCap];
 
-  __shared__ int s_unit;
-  const int n_tiles = p.hdr[0];
-  const int xcd = (int)blockIdx.x & 7;  // workgroups are dispatched to the 8 XCDs round-robin
+  __shared__ int s_unit, s_slot;
 
   // ---- persistent: take units from this XCD's queue, then steal from the others
   for (;;) {
-  if (threadIdx.x == 0) {
-    int u = -1;
-    for (int k = 0; k < 8 && u < 0; ++k) {
-      const int y = (xcd + k) & 7;
-      const int first = p.hdr[8 + y], len = p.hdr[9 + y] - first;
-      if (len <= 0 || __hip_atomic_load(p.ctr + y * kCtrStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= len)
-        continue;
-      const int i = atomicAdd(p.ctr + y * kCtrStride, 1);
-      if (i < len) u = p.order[first + i];
-    }
-    s_unit = u;
+  if (threadIdx.x < 64) {
+    const int u = pf_claim(p);
+    if (threadIdx.x == 0) s_unit = u;
   }
   __syncthreads();
-  const int unit = s_unit;
+  const int unit = uniform(s_unit);
   __syncthreads();
   if (unit < 0) break;
-  const int h = unit / n_tiles;
-  const int tile = unit - h * n_tiles;
-  const int2 te = p.tiles[tile];
-  const int b = te.x, row0 = te.y;
+  const PfUnit un = pf_unit(p, unit);
+  const int h = un.h, b = un.b, row0 = un.row0;
+  s_slot = un.n > 1 ? un.slot : -1;  // for the epilogue: no register is held for it
 
   const int tid = threadIdx.x;
   const int lane = lane_id();
@@ -139,6 +243,8 @@ __global__ __launch_bounds__(64 * pf_waves(D)) void prefill_kernel(PrefillParams
   const int kv_end = p.causal ? min(kv_len, kv_len - qo_len + max_tok + 1) : kv_len;
   const int mask_from = p.causal ? (kv_len - qo_len + min_tok + 1) : kv_len;
   const int n_kt = kv_end > 0 ? (kv_end + KEYS - 1) / KEYS : 0;
+  // key steps of this unit: all of the tile's, or its piece's share
+  const int kt0 = un.n > 1 ? un.k * n_kt / un.n : 0, kt1 = un.n > 1 ? (un.k + 1) * n_kt / un.n : n_kt;
 
   float kscale = 1.f, vscale = 1.f;
   if constexpr (FP8) {
@@ -400,9 +506,9 @@ __global__ __launch_bounds__(64 * pf_waves(D)) void prefill_kernel(PrefillParams
   // no page or slot arithmetic.  Loads past the last tile repeat the last
   // tile, so the steady loop has no conditional loads and the compiler's
   // vmcnt waits stay exact.
-  for (c0 = 0; c0 * KEYS < kv_end; c0 += kPfTileCap) {
+  for (c0 = kt0; c0 < kt1; c0 += kPfTileCap) {
     const int t0 = c0;
-    const int t1 = min(n_kt, c0 + kPfTileCap);
+    const int t1 = min(kt1, c0 + kPfTileCap);
     __syncthreads();
     for (int e = tid; e < 2 * (t1 - t0); e += THREADS) {
       const int key = min((t0 + (e >> 1)) * KEYS + 16 * (e & 1), key_cap);
@@ -482,10 +588,18 @@ __global__ __launch_bounds__(64 * pf_waves(D)) void prefill_kernel(PrefillParams
   }
 
   // ---- epilogue: lane holds dims 16*jj + 4*grp + r of its row
+  const int slot = uniform(s_slot);
 #pragma unroll
   for (int rg = 0; rg < RG; ++rg) {
     const float l_tot = rows4_sum(l_run[rg]);
     const float inv = l_tot > 0.f ? vscale / l_tot : (l_tot == 0.f ? 0.f : __builtin_nanf(""));  // NaN: row stays NaN
+    if (slot >= 0) {  // a piece of a split tile: a partial for the merge
+      if (row0 + WROWS * wave + 16 * rg < rows_total)
+        pf_put_part<VW, C::ROWS>(p, slot, RG * wave + rg, acc[rg], inv,
+                                 l_tot > 0.f ? m_run[rg] * sl2 + fast_log2(l_tot)
+                                             : (l_tot == 0.f ? kNegInf : __builtin_nanf("")));
+      continue;
+    }
     const int n = row0 + WROWS * wave + 16 * rg + col;
     if (n >= rows_total) continue;
     const int tok = n / G, g = n - tok * G;
@@ -498,15 +612,7 @@ __global__ __launch_bounds__(64 * pf_waves(D)) void prefill_kernel(PrefillParams
     }
   }
   }  // unit loop
-  // The last workgroup to finish resets the queues for the next run with
-  // this plan (every other workgroup has taken its last unit by then).
-  if (threadIdx.x == 0) {
-    __threadfence();
-    if (atomicAdd(p.ctr + 8 * kCtrStride, 1) == (int)gridDim.x - 1) {
-#pragma unroll
-      for (int y = 0; y < 9; ++y) __hip_atomic_store(p.ctr + y * kCtrStride, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
+  pf_done(p);
 }
 
 // head_dim 128 launches, defined in mi_prefill_d128.hip

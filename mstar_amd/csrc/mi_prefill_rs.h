@@ -58,10 +58,8 @@ __global__ __launch_bounds__(512) void prefill_rs_kernel(PrefillParams p) {
   // one uint4) and each row's rescale factor, double-buffered by step parity
   __shared__ uint4 lds_p[2][4][RGP][64];
   __shared__ float lds_alpha[2][4][RGP][64];
-  __shared__ int s_unit;
+  __shared__ int s_unit, s_slot;
 
-  const int n_tiles = p.hdr[0];
-  const int xcd = (int)blockIdx.x & 7;
   const int tid = threadIdx.x;
   const int lane = lane_id();
   const int wave = uniform(tid >> 6);
@@ -77,25 +75,17 @@ __global__ __launch_bounds__(512) void prefill_rs_kernel(PrefillParams p) {
   auto run = [&](auto role) {
     constexpr bool S = decltype(role)::value;
     for (;;) {
-      if (tid == 0) {
-        int u = -1;
-        for (int k = 0; k < 8 && u < 0; ++k) {
-          const int y = (xcd + k) & 7;
-          const int first = p.hdr[8 + y], len = p.hdr[9 + y] - first;
-          if (len <= 0 || __hip_atomic_load(p.ctr + y * kCtrStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= len)
-            continue;
-          const int i = atomicAdd(p.ctr + y * kCtrStride, 1);
-          if (i < len) u = p.order[first + i];
-        }
-        s_unit = u;
+      if (wave == 0) {
+        const int u = pf_claim(p);
+        if (tid == 0) s_unit = u;
       }
       __syncthreads();
-      const int unit = s_unit;
+      const int unit = uniform(s_unit);
       __syncthreads();
       if (unit < 0) break;
-      const int h = unit / n_tiles;
-      const int2 te = p.tiles[unit - h * n_tiles];
-      const int b = te.x, row0 = te.y;
+      const PfUnit un = pf_unit(p, unit);
+      const int h = un.h, b = un.b, row0 = un.row0;
+      s_slot = un.n > 1 ? un.slot : -1;  // for the epilogue: no register is held for it
       const int qo_start = p.qo_indptr[b];
       const int qo_len = p.qo_indptr[b + 1] - qo_start;
       const int page_base = p.kv_indptr[b];
@@ -129,6 +119,8 @@ __global__ __launch_bounds__(512) void prefill_rs_kernel(PrefillParams p) {
       const int kv_end = p.causal ? min(kv_len, kv_len - qo_len + max_tok + 1) : kv_len;
       const int mask_from = p.causal ? (kv_len - qo_len + min_tok + 1) : kv_len;
       const int n_kt = kv_end > 0 ? (kv_end + KEYS - 1) / KEYS : 0;
+      // key steps of this unit: all of the tile's, or its piece's share
+      const int kt0 = un.n > 1 ? un.k * n_kt / un.n : 0, kt1 = un.n > 1 ? (un.k + 1) * n_kt / un.n : n_kt;
 
       float kscale = 1.f, vscale = 1.f;
       if constexpr (FP8) {
@@ -440,9 +432,9 @@ __global__ __launch_bounds__(512) void prefill_rs_kernel(PrefillParams p) {
         // of tile ii-1, then every wave's direct loads of tile ii+2 (ring stage
         // (ii+2) % 4); before the barrier each wave's loads of K of tile ii+1
         // and V of tile ii have landed (and are visible to all after it).
-        for (c0 = 0; c0 * KEYS < kv_end; c0 += CAP) {
+        for (c0 = kt0; c0 < kt1; c0 += CAP) {
           const int t0 = c0;
-          const int t1 = min(n_kt, c0 + CAP);
+          const int t1 = min(kt1, c0 + CAP);
           __syncthreads();
           for (int e = tid; e < 2 * (t1 - t0); e += THREADS) {
             const int key = min((t0 + (e >> 1)) * KEYS + 16 * (e & 1), key_cap);
@@ -497,9 +489,9 @@ __global__ __launch_bounds__(512) void prefill_rs_kernel(PrefillParams p) {
       } else {
         // as prefill_kernel: step T stores tile T+1 into the stage tile T-2 used
         // and loads tile T+1+NB into registers
-        for (c0 = 0; c0 * KEYS < kv_end; c0 += kPfTileCap) {
+        for (c0 = kt0; c0 < kt1; c0 += kPfTileCap) {
           const int t0 = c0;
-          const int t1 = min(n_kt, c0 + kPfTileCap);
+          const int t1 = min(kt1, c0 + kPfTileCap);
           __syncthreads();
           for (int e = tid; e < 2 * (t1 - t0); e += THREADS) {
             const int key = min((t0 + (e >> 1)) * KEYS + 16 * (e & 1), key_cap);
@@ -543,12 +535,29 @@ __global__ __launch_bounds__(512) void prefill_rs_kernel(PrefillParams p) {
         }
       }
 
-      // ---- epilogue: the S-role publishes its row sums, the O-role writes the rows
+      // ---- epilogue: the O-role writes the rows.  For a piece of a split tile
+      // the S-role first hands its running max over LDS (the rescale buffer of
+      // the parity that the last tile's P.V does not read).
+      const int slot = uniform(s_slot);
+      if (slot >= 0) {
+        if constexpr (S) {
+#pragma unroll
+          for (int rg = 0; rg < RGP; ++rg) lds_alpha[kt1 & 1][pr][rg][lane] = m_run[rg] * sl2;
+        }
+        __syncthreads();
+      }
       if constexpr (!S) {
 #pragma unroll
         for (int rg = 0; rg < RGP; ++rg) {
           const float l_tot = rows4_sum(l_run[rg]);
           const float inv = l_tot > 0.f ? vscale / l_tot : (l_tot == 0.f ? 0.f : __builtin_nanf(""));
+          if (slot >= 0) {  // a piece of a split tile: a partial for the merge
+            if (row0 + PROWS * pr + 16 * rg < rows_total)
+              pf_put_part<VW, C::ROWS>(p, slot, RGP * pr + rg, R[rg], inv,
+                                       l_tot > 0.f ? lds_alpha[kt1 & 1][pr][rg][lane] + fast_log2(l_tot)
+                                                   : (l_tot == 0.f ? kNegInf : __builtin_nanf("")));
+            continue;
+          }
           const int nrow = row0 + PROWS * pr + 16 * rg + col;
           if (nrow >= rows_total) continue;
           const int tok = nrow / G, g = nrow - tok * G;
@@ -568,13 +577,7 @@ __global__ __launch_bounds__(512) void prefill_rs_kernel(PrefillParams p) {
     run(std::true_type{});
   else
     run(std::false_type{});
-  if (tid == 0) {
-    __threadfence();
-    if (atomicAdd(p.ctr + 8 * kCtrStride, 1) == (int)gridDim.x - 1) {
-#pragma unroll
-      for (int y = 0; y < 9; ++y) __hip_atomic_store(p.ctr + y * kCtrStride, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
+  pf_done(p);
 }
 
 }  // namespace mi
