@@ -327,6 +327,196 @@ __global__ __launch_bounds__(256) void attend_f32_kernel(DecodeParams p, F32Tile
   }
 }
 
+// Prefill with K and V shared by the workgroup: 64 rows of one (tile,
+// kv-head), 16 per wavefront, and every wavefront goes over all the keys its
+// rows can see.  Steps of KT keys (64 rows of K and V together are 32 KB at
+// any head_dim) go through two LDS stages, filled from registers that were
+// loaded a step ahead, page ids a step before that; each 16-byte LDS read of a
+// K or V fragment feeds four MFMAs.  attend_f32_kernel<D, true> reads each K/V
+// row from L2 once per 16 rows and keys' quarter instead: on 4 prefixes of
+// 800-1000 tokens at 8 q / 1 kv / 256 its 3.3 GB of L2 reads, not the MFMAs,
+// set the time.  Here the matrix cores are busy 70% of the time: 382 -> 268 us on 4 x 900
+// keys, 69 -> 99 TFLOP/s (without the softmax, with fragments read six ahead or
+// with two key groups per workgroup in opposite phase no faster).
+// S^T, the softmax and O^T use the same operand layouts as there (S^T in two
+// chains over the head_dim); V rows past kv_len are stored as zeros.
+template <int D>
+__global__ __launch_bounds__(256, 2) void prefill_f32_kernel(DecodeParams p, F32Tiles pt) {
+  constexpr int VW = D / 16, NV = VW / 4, KQ = D / 4, RUN = lane_run(D, 4);
+  constexpr int KT = 16 * (256 / D), NS = KT / 16;  // keys and 16-key groups per step
+  constexpr int KRS = D * 4 + 16;   // LDS row stride of K: rows 4 banks apart for the fragment reads
+  constexpr int CPR = D / 4;        // 16-byte chunks per row
+  constexpr int NL = KT * CPR / 256;  // chunks of K (and of V) per thread
+  constexpr int CPG = 16 * CPR / 256;  // of them in one 16-key group
+  constexpr float kNegInf = -__builtin_inff();
+  __shared__ __attribute__((aligned(16))) uint8_t lds_k[2][KT * KRS];
+  __shared__ __attribute__((aligned(16))) uint8_t lds_v[2][KT * D * 4];
+
+  const int tid = (int)threadIdx.x, lane = lane_id(), wave = uniform(tid >> 6);
+  const int col = lane & 15, grp = lane >> 4;
+  const int nkv = p.num_kv_heads, G = p.group, ps = p.page_size;
+  const int bpt = pt.tile_rows / 64;  // 64-row blocks per tile
+  const int x = (int)blockIdx.x;
+  const int j = x % bpt, rest = x / bpt, t_idx = rest / nkv;
+  const int h = uniform(rest - t_idx * nkv);
+  if (t_idx >= pt.hdr[0]) return;  // uniform
+  const int2 tile = pt.tiles[t_idx];
+  const int b = uniform(tile.x), row_wg = uniform(tile.y + 64 * j);
+  const int page_base = p.kv_indptr[b];
+  const int np = p.kv_indptr[b + 1] - page_base;
+  const int kv_len = (np - 1) * ps + p.last_page_len[b];
+  const int qo_start = p.qo_indptr[b], qo_len = p.qo_indptr[b + 1] - qo_start;
+  const int rows_wg = min(qo_len * G - row_wg, 64);
+  if (rows_wg <= 0) return;  // uniform: past the request's last row
+  const int last_qtok = (row_wg + rows_wg - 1) / G;
+  const int kv_end = p.causal ? min(kv_len, kv_len - qo_len + last_qtok + 1) : kv_len;
+  const int steps = kv_end > 0 ? (kv_end + KT - 1) / KT : 0;
+
+  const int row = row_wg + 16 * wave + col, qtok = row / G, g = row - qtok * G;
+  const bool row_valid = row < qo_len * G;
+  int lim = p.causal ? (kv_len - qo_len + qtok) : (kv_len - 1);
+  lim = min(lim, kv_len - 1);
+  const int mask_from = p.causal ? (kv_len - qo_len + row_wg / G + 1) : kv_len;  // keys >= this need a row check
+
+  float4 qf[KQ / 4];
+  {
+    const float* qrow = (const float*)p.q + (int64_t)(qo_start + qtok) * p.q_stride_tok +
+                        (int64_t)(h * G + g) * p.q_stride_head + KQ * grp;
+#pragma unroll
+    for (int i = 0; i < KQ / 4; ++i) qf[i] = row_valid ? *(const float4*)(qrow + 4 * i) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  const float sl2 = p.scale_log2;
+
+  // loader: chunk tid + 256 i of the step's K rows and of its V rows; a
+  // wavefront's 64 chunks lie in one 16-key group, hence in one page
+  const uint8_t* kvb = (const uint8_t*)p.kv + (int64_t)h * p.head_stride * 4;
+  const int64_t tok_bytes = p.token_stride * 4, page_bytes = p.page_stride * 4, kvhalf = p.kv_stride * 4;
+  const int key_cap = np * ps - 16;  // last group inside the request's pages
+  int pg[NS], slot[NS];  // page and slot of the groups of the step to load next
+  auto find_pages = [&](int t) {
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+      const int key = min(t * KT + 16 * k, key_cap), pidx = (int)((unsigned)key / (unsigned)ps);
+      pg[k] = p.kv_indices[page_base + pidx];
+      slot[k] = key - pidx * ps;
+    }
+  };
+  f32x4 rk[NL], rv[NL];
+  auto load_step = [&]() {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int c = tid + 256 * i, r = (c / CPR) & 15, k = i / CPG;
+      const uint8_t* src = kvb + (int64_t)pg[k] * page_bytes + (int64_t)(slot[k] + r) * tok_bytes + 16 * (c % CPR);
+      rk[i] = *(const f32x4*)src;
+      rv[i] = *(const f32x4*)(src + kvhalf);
+    }
+  };
+  auto store_step = [&](int t, int st) {
+    const bool tail = (t + 1) * KT > kv_len;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int c = tid + 256 * i, r = c / CPR;
+      const bool past = tail && t * KT + r >= kv_len;  // slots past the end hold stale data
+      *(f32x4*)(lds_k[st] + r * KRS + 16 * (c % CPR)) = rk[i];
+      *(f32x4*)(lds_v[st] + r * D * 4 + 16 * (c % CPR)) = past ? f32x4{0.f, 0.f, 0.f, 0.f} : rv[i];
+    }
+  };
+
+  f32x4 acc[VW];
+#pragma unroll
+  for (int m = 0; m < VW; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = kNegInf, l_run = 0.f;
+
+  auto compute = [&](int t, int st) {
+    float sv[NS][4];
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+      f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+      const float4* krun = (const float4*)(lds_k[st] + (16 * k + col) * KRS + KQ * grp * 4);
+#pragma unroll
+      for (int i = 0; i < KQ / 4; ++i) {
+        const float4 a = krun[i];
+        s0 = mma_f32(a.x, qf[i].x, s0);
+        s1 = mma_f32(a.y, qf[i].y, s1);
+        s0 = mma_f32(a.z, qf[i].z, s0);
+        s1 = mma_f32(a.w, qf[i].w, s1);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sv[k][r] = (s0[r] + s1[r]) * sl2;
+    }
+    if ((t + 1) * KT > mask_from) {
+#pragma unroll
+      for (int k = 0; k < NS; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (t * KT + 16 * k + 4 * grp + r > lim) sv[k][r] = kNegInf;
+    }
+    float ml = kNegInf;  // this lane's share of the row
+#pragma unroll
+    for (int k = 0; k < NS; ++k) ml = fmaxf(ml, fmaxf(fmaxf(sv[k][0], sv[k][1]), fmaxf(sv[k][2], sv[k][3])));
+    // The running max is raised only when a score exceeds it by more than 8:
+    // probabilities then stay below 2^8, which costs fp32 no precision, and most
+    // steps need neither the row max across lanes nor a rescale of O.
+    if (__builtin_amdgcn_ballot_w64(ml > m_run + 8.f)) {
+      const float m_new = fmaxf(m_run, rows4_max(ml));
+      const float alpha = m_new > m_run ? fast_exp2(m_run - m_new) : 1.f;
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int m = 0; m < VW; ++m) acc[m] *= alpha;
+    }
+    const float m_use = m_run == kNegInf ? 0.f : m_run;
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sv[k][r] = fast_exp2(sv[k][r] - m_use);
+      l_run += (sv[k][0] + sv[k][1]) + (sv[k][2] + sv[k][3]);
+    }
+#pragma unroll
+    for (int k = 0; k < NS; ++k)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const uint8_t* vrow = lds_v[st] + (16 * k + 4 * grp + r) * D * 4 + 16 * col;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {  // elements 4i..4i+3 of the lane: dims dim_of(RUN, col, 4i)
+          const float4 a = *(const float4*)(vrow + 256 * i);
+          acc[4 * i] = mma_f32(a.x, sv[k][r], acc[4 * i]);
+          acc[4 * i + 1] = mma_f32(a.y, sv[k][r], acc[4 * i + 1]);
+          acc[4 * i + 2] = mma_f32(a.z, sv[k][r], acc[4 * i + 2]);
+          acc[4 * i + 3] = mma_f32(a.w, sv[k][r], acc[4 * i + 3]);
+        }
+      }
+  };
+  static_assert(RUN == 4, "a lane's dims: one float4 per 64");
+
+  if (steps > 0) {
+    find_pages(0);
+    load_step();
+    find_pages(1);
+    store_step(0, 0);
+    __syncthreads();
+    for (int t = 0; t < steps; ++t) {
+      if (t + 1 < steps) {
+        load_step();  // step t + 1
+        find_pages(t + 2);
+      }
+      compute(t, t & 1);
+      if (t + 1 < steps) store_step(t + 1, (t + 1) & 1);  // the stage of step t - 1
+      __syncthreads();
+    }
+  }
+  const float L = rows4_sum(l_run);
+  const float inv = L > 0.f ? 1.f / L : (L == 0.f ? 0.f : __builtin_nanf(""));  // NaN L: keep the row NaN
+  if (!row_valid) return;
+  float* dst = (float*)p.out + (int64_t)(qo_start + qtok) * p.out_stride_tok + (int64_t)(h * G + g) * p.out_stride_head;
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      *(float4*)(dst + dim_of(RUN, 4 * grp + r, 4 * i)) = make_float4(acc[4 * i][r] * inv, acc[4 * i + 1][r] * inv,
+                                                                       acc[4 * i + 2][r] * inv, acc[4 * i + 3][r] * inv);
+}
+
 template <int D, bool PREFILL>
 static void launch_f32(const DecodeParams& dp, const F32Tiles& pt, int grid, hipStream_t stream) {
   hipLaunchKernelGGL((attend_f32_kernel<D, PREFILL>), dim3(grid), dim3(256), 0, stream, dp, pt);
@@ -348,9 +538,28 @@ int f32_attend_launch(const DecodeParams& dp, int head_dim, int grid, hipStream_
   return dispatch_f32<false>(dp, F32Tiles{nullptr, nullptr, 0}, head_dim, grid, stream);
 }
 
+// From how many of its 64-row blocks per CU on the shared-K/V kernel is the
+// faster one: a block of it is a long serial job (900 keys at head_dim 256:
+// 155 us), where the other kernel has four times the workgroups.  us, other ->
+// shared, 900 keys: head_dim 256, 113 blocks 96 -> 161, 225 192 -> 159, 450
+// 382 -> 268; head_dim 128, 114 53 -> 82, 226 105 -> 82, 450 212 -> 146;
+// head_dim 64, 228 46 -> 48, 452 86 -> 78, 900 185 -> 155.
+static double shared_from(int head_dim) { return head_dim == 64 ? 1.5 : 0.8; }
+
 int f32_prefill_launch(const DecodeParams& dp, const int32_t* tile_hdr, const int2* tiles, int max_tiles,
-                       int tile_rows, int head_dim, hipStream_t stream) {
-  if (tile_rows <= 0 || tile_rows % kRows) return MI_ERR_INVALID;
+                       int tile_rows, int64_t rows, int head_dim, hipStream_t stream) {
+  if (tile_rows <= 0 || tile_rows % 64) return MI_ERR_INVALID;
+  const int64_t blocks = (int64_t)max_tiles * dp.num_kv_heads * (tile_rows / 64);
+  if ((double)rows / 64 * dp.num_kv_heads >= shared_from(head_dim) * device_cu_count() && blocks <= 0x7fffffff) {
+    const F32Tiles pt{tile_hdr, tiles, tile_rows};
+    switch (head_dim) {
+      case 64: hipLaunchKernelGGL((prefill_f32_kernel<64>), dim3((int)blocks), dim3(256), 0, stream, dp, pt); break;
+      case 128: hipLaunchKernelGGL((prefill_f32_kernel<128>), dim3((int)blocks), dim3(256), 0, stream, dp, pt); break;
+      case 256: hipLaunchKernelGGL((prefill_f32_kernel<256>), dim3((int)blocks), dim3(256), 0, stream, dp, pt); break;
+      default: return MI_ERR_UNSUPPORTED;
+    }
+    return MI_OK;
+  }
   const int64_t grid = (int64_t)max_tiles * dp.num_kv_heads * (tile_rows / kRows);
   if (grid <= 0) return MI_OK;
   if (grid > 0x7fffffff) return MI_ERR_UNSUPPORTED;

@@ -116,10 +116,11 @@ struct DecodeParams {
 // (mi_f32.hip), and the merge with fp32 output (mi_decode.hip).
 int f32_attend_launch(const DecodeParams& dp, int head_dim, int grid, hipStream_t stream);
 int merge_launch(const DecodeParams& dp, int head_dim, int out_dtype, int batch, hipStream_t stream);
-// fp32 ragged prefill over the prefill plan's tile list: one workgroup per
-// (tile, kv-head, 16-row block).
+// fp32 ragged prefill over the prefill plan's tile list, one workgroup per
+// (tile, kv-head, block of 16 or 64 rows); rows: the most (token, q-head) rows
+// the batch can have.
 int f32_prefill_launch(const DecodeParams& dp, const int32_t* tile_hdr, const int2* tiles, int max_tiles,
-                       int tile_rows, int head_dim, hipStream_t stream);
+                       int tile_rows, int64_t rows, int head_dim, hipStream_t stream);
 
 int decode_run_impl(const void* q, int32_t q_dtype, int64_t q_stride_token, int64_t q_stride_head,
                     const mi_paged_kv* kv, const int32_t* qo_indptr, const int32_t* kv_indptr,

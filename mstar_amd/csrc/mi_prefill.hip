@@ -752,7 +752,7 @@ static int prefill_run_impl(const void* q, int32_t q_dtype, int64_t q_stride_tok
   }
   if (!(phases & kPhaseTiles)) return MI_OK;
   const uint8_t* ws = (const uint8_t*)workspace;
-  if (q_dtype == MI_F32) {  // fp32 KV: one workgroup per (tile, kv-head, 16-row block) of the plan's tiles
+  if (q_dtype == MI_F32) {  // fp32 KV: the plan's tiles by blocks of rows
     DecodeParams dp{};
     dp.q = q;
     dp.q_stride_tok = q_stride_token;
@@ -775,7 +775,7 @@ static int prefill_run_impl(const void* q, int32_t q_dtype, int64_t q_stride_tok
     dp.causal = causal ? 1 : 0;
     dp.scale_log2 = sm_scale * 1.4426950408889634f;
     st = f32_prefill_launch(dp, (const int32_t*)(ws + L.hdr), (const int2*)(ws + L.tiles), L.max_tiles,
-                            pf_rows(D), D, s);
+                            pf_rows(D), (int64_t)max_qo_tokens * G, D, s);
     if (st != MI_OK) return st;
     MI_CHECK_LAUNCH();
     return MI_OK;
