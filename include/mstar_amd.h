@@ -294,6 +294,27 @@ int mi_prefill_plan(const int32_t* qo_indptr, const int32_t* kv_indptr,
                     int32_t num_kv_heads, int32_t head_dim, int64_t* token_to_page,
                     int64_t* token_to_cache, int32_t token_map_len, void* workspace,
                     int64_t workspace_bytes, void* stream);
+/* mi_prefill_plan (mi_decode_plan below) for index arrays in host memory: the
+ * four (three) arrays travel in the launch argument, and the launch writes them
+ * to the device arrays that the run call will read before it plans, so that a
+ * step with few pages needs no copy of its own.  num_indices: elements of
+ * kv_indices.  At most MI_PLAN_HOST_ARGS int32 values in all
+ * (MI_ERR_UNSUPPORTED beyond: copy them and call the other entry point); the
+ * host arrays are not read after the call returns.  No counterpart in the
+ * reference, which copies its index tensors one by one. */
+#define MI_PLAN_HOST_ARGS 800
+int mi_prefill_plan_host(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host,
+                         const int32_t* kv_indices_host, const int32_t* last_page_len_host,
+                         int32_t num_indices, int32_t* qo_indptr, int32_t* kv_indptr, int32_t* kv_indices,
+                         int32_t* last_page_len, int32_t batch, int32_t max_qo_tokens, int32_t page_size,
+                         int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim, int64_t* token_to_page,
+                         int64_t* token_to_cache, int32_t token_map_len, void* workspace,
+                         int64_t workspace_bytes, void* stream);
+int mi_decode_plan_host(const int32_t* kv_indptr_host, const int32_t* kv_indices_host,
+                        const int32_t* last_page_len_host, int32_t num_indices, int32_t* kv_indptr,
+                        int32_t* kv_indices, int32_t* last_page_len, int32_t batch, int32_t page_size,
+                        int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim, int64_t* kv_locations,
+                        void* workspace, int64_t workspace_bytes, void* stream);
 int mi_prefill_run(const void* q, int32_t q_dtype, int64_t q_stride_token, int64_t q_stride_head,
                    const mi_paged_kv* kv, const int32_t* qo_indptr, const int32_t* kv_indptr,
                    const int32_t* kv_indices, const int32_t* last_page_len, int32_t batch,

@@ -93,6 +93,10 @@ SIGNATURES = {
     "mi_block_table_update": (ctypes.c_int, [_P, _I64, _P, _P, _P, _I32, _P]),
     "mi_decode_workspace_bytes": (_I64, [_I32, _I32, _I32, _I32]),
     "mi_decode_plan": (ctypes.c_int, [_P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _P, _P, _I64, _P]),
+    "mi_decode_plan_host": (
+        ctypes.c_int,
+        [_P, _P, _P, _I32, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _P, _P, _I64, _P],
+    ),
     "mi_decode_run": (
         ctypes.c_int,
         [_P, _I32, _I64, _I64, ctypes.POINTER(MiPagedKV), _P, _P, _P, _P, _I32, _I32, _I32, _F32,
@@ -122,6 +126,10 @@ SIGNATURES = {
     "mi_prefill_plan": (
         ctypes.c_int,
         [_P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _P, _P, _I32, _P, _I64, _P],
+    ),
+    "mi_prefill_plan_host": (
+        ctypes.c_int,
+        [_P, _P, _P, _P, _I32, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _P, _P, _I32, _P, _I64, _P],
     ),
     "mi_prefill_run": (
         ctypes.c_int,
@@ -258,6 +266,7 @@ def _event_create(device: torch.device) -> int:
     return ev.value
 
 
+PLAN_HOST_ARGS = 800  # MI_PLAN_HOST_ARGS: int32 values of host index arrays a plan call passes as a kernel argument
 PACK_HOST_META = 768  # MI_PACK_HOST_META: int32 values of step metadata always passed as a kernel argument
 PACK_HOST_META_MAX = 4096  # MI_PACK_HOST_META_MAX: up to this many when the step fits the argument's compact form
 

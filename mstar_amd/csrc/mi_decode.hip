@@ -92,6 +92,17 @@ SplitLayout split_layout(int32_t batch, int32_t nkv, int32_t head_dim, int64_t w
 
 __global__ __launch_bounds__(1024) void decode_plan_kernel(PlanParams p) { decode_plan_body(p); }
 
+// The index arrays in the argument: they are in LDS for the plan, so its
+// chain of reads does not wait for memory either.
+__global__ __launch_bounds__(1024) void decode_plan_host_kernel(PlanParams p, HostIndices m) {
+  __shared__ int32_t s_idx[MI_PLAN_HOST_ARGS];
+  host_indices_copy(m, s_idx, true);
+  p.kv_indptr = s_idx;
+  p.kv_indices = s_idx + m.end[0];
+  p.last_page_len = s_idx + m.end[1];
+  decode_plan_body(p);
+}
+
 // ---------------------------------------------------------------- decode
 
 // Per-lane registers of one 16-token tile.
@@ -650,6 +661,22 @@ int decode_plan_impl(const int32_t* qo_indptr, const int32_t* kv_indptr, const i
   return MI_OK;
 }
 
+static int decode_plan_host_impl(const int32_t* const* src, int32_t num_indices, int32_t* const* dst, int32_t batch,
+                                 int32_t page_size, int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim,
+                                 int64_t* kv_locations, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
+  PlanParams pp{};
+  int st = decode_plan_params(nullptr, dst[0], dst[1], dst[2], batch, page_size, num_qo_heads, num_kv_heads, head_dim,
+                              kv_locations, workspace, workspace_bytes, 0, &pp);
+  if (st != MI_OK) return st;
+  const int32_t len[3] = {batch + 1, num_indices, batch};
+  HostIndices m;
+  st = host_indices(src, len, dst, 3, &m);
+  if (st != MI_OK) return st;
+  hipLaunchKernelGGL(decode_plan_host_kernel, dim3(1), dim3(1024), 0, stream, pp, m);
+  MI_CHECK_LAUNCH();
+  return MI_OK;
+}
+
 template <typename MT, bool FP8, int D>
 static void launch_decode(const DecodeParams& dp, int grid, int batch, int phases, hipStream_t stream) {
   if (phases & kPhaseAttend)
@@ -817,6 +844,17 @@ int mi_decode_plan(const int32_t* qo_indptr, const int32_t* kv_indptr, const int
   return mi::decode_plan_impl(qo_indptr, kv_indptr, kv_indices, last_page_len, batch, page_size,
                               num_qo_heads, num_kv_heads, head_dim, kv_locations, workspace,
                               workspace_bytes, 0, (hipStream_t)stream);
+}
+
+int mi_decode_plan_host(const int32_t* kv_indptr_host, const int32_t* kv_indices_host,
+                        const int32_t* last_page_len_host, int32_t num_indices, int32_t* kv_indptr,
+                        int32_t* kv_indices, int32_t* last_page_len, int32_t batch, int32_t page_size,
+                        int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim, int64_t* kv_locations,
+                        void* workspace, int64_t workspace_bytes, void* stream) {
+  const int32_t* const src[3] = {kv_indptr_host, kv_indices_host, last_page_len_host};
+  int32_t* const dst[3] = {kv_indptr, kv_indices, last_page_len};
+  return mi::decode_plan_host_impl(src, num_indices, dst, batch, page_size, num_qo_heads, num_kv_heads, head_dim,
+                                   kv_locations, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 #define MI_DECODE_ARGS                                                                           \

@@ -72,6 +72,50 @@ int decode_plan_params(const int32_t* qo_indptr, const int32_t* kv_indptr, const
                        int64_t* kv_locations, void* workspace, int64_t workspace_bytes,
                        int64_t ws_offset, PlanParams* out, bool ragged_pair = false);
 
+// Index arrays of a plan call as a kernel argument (mi_decode_plan_host,
+// mi_prefill_plan_host): one after the other, and where the device copies go.
+constexpr int kHostParts = 4;
+struct HostIndices {
+  int32_t v[MI_PLAN_HOST_ARGS];
+  int32_t end[kHostParts];  // part k is v[end[k - 1], end[k])
+  int32_t* dst[kHostParts];
+};
+// Fills one; MI_ERR_UNSUPPORTED when the parts do not fit.
+inline int host_indices(const int32_t* const* src, const int32_t* len, int32_t* const* dst, int parts, HostIndices* out) {
+  int64_t at = 0;
+  for (int k = 0; k < kHostParts; ++k) {
+    const int32_t n = k < parts ? len[k] : 0;
+    if (n < 0 || (n > 0 && (!src[k] || !dst[k]))) return MI_ERR_INVALID;
+    if (at + n > MI_PLAN_HOST_ARGS) return MI_ERR_UNSUPPORTED;
+    for (int32_t i = 0; i < n; ++i) out->v[at + i] = src[k][i];
+    at += n;
+    out->end[k] = (int32_t)at;
+    out->dst[k] = k < parts ? dst[k] : nullptr;
+  }
+  return MI_OK;
+}
+// The workgroup's copy of the argument in LDS, and, by one workgroup of the
+// launch (write), the device arrays.
+__device__ __forceinline__ void host_indices_copy(const HostIndices& m, int32_t* s_idx, bool write) {
+  const int total = m.end[kHostParts - 1];
+  for (int i = (int)threadIdx.x; i < total; i += (int)blockDim.x) {
+    const int32_t v = m.v[i];
+    s_idx[i] = v;
+    if (write) {
+      int first = 0;
+      int32_t* d = m.dst[0];
+#pragma unroll
+      for (int k = 1; k < kHostParts; ++k)
+        if (i >= m.end[k - 1]) {
+          first = m.end[k - 1];
+          d = m.dst[k];
+        }
+      d[i - first] = v;
+    }
+  }
+  __syncthreads();
+}
+
 enum : int { kPhaseAttend = 1, kPhaseMerge = 2 };
 
 // The attention kernels move q / out rows and KV rows in 16-byte pieces: a

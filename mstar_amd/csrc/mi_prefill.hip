@@ -521,6 +521,31 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(PfPlanArgs a, PlanPa
   }
 }
 
+// The index arrays in the argument: every workgroup plans from its own copy in
+// LDS, workgroup 0 also writes the device arrays.
+__global__ __launch_bounds__(1024) void prefill_plan_host_kernel(PfPlanArgs a, PlanParams d, TokenMapArgs m, HostIndices h) {
+  __shared__ int32_t s_idx[MI_PLAN_HOST_ARGS];
+  host_indices_copy(h, s_idx, blockIdx.x == 0);
+  const int32_t *qo = s_idx, *kvp = s_idx + h.end[0], *idx = s_idx + h.end[1], *last = s_idx + h.end[2];
+  if (blockIdx.x == 0) {
+    a.qo_indptr = qo;
+    a.kv_indptr = kvp;
+    a.last_page_len = last;
+    prefill_plan_body(a);
+  } else if (blockIdx.x == 1) {
+    d.qo_indptr = qo;
+    d.kv_indptr = kvp;
+    d.kv_indices = idx;
+    d.last_page_len = last;
+    decode_plan_body(d);
+  } else {
+    m.qo_indptr = qo;
+    m.kv_indptr = kvp;
+    m.kv_indices = idx;
+    m.last_page_len = last;
+    token_map_body(m, ((int)blockIdx.x - 2) * 1024 + (int)threadIdx.x);
+  }
+}
 
 template <typename MT, bool FP8>
 static int launch_prefill(const PrefillParams& pp, int head_dim, int grid, hipStream_t stream) {
@@ -642,13 +667,14 @@ extern "C" int32_t mi_prefill_short_rows(int32_t batch, int32_t num_qo_heads, in
   return pair_short_rows(pair_heads(nullptr, batch, num_kv_heads, G, head_dim, true));
 }
 
-extern "C" int mi_prefill_plan(const int32_t* qo_indptr, const int32_t* kv_indptr,
-                               const int32_t* kv_indices, const int32_t* last_page_len, int32_t batch,
-                               int32_t max_qo_tokens, int32_t page_size, int32_t num_qo_heads,
-                               int32_t num_kv_heads, int32_t head_dim, int64_t* token_to_page,
-                               int64_t* token_to_cache, int32_t token_map_len, void* workspace,
-                               int64_t workspace_bytes, void* stream) {
-  using namespace mi;
+namespace mi {
+
+// host: the index arrays in the launch argument, or NULL
+static int prefill_plan_impl(const int32_t* qo_indptr, const int32_t* kv_indptr, const int32_t* kv_indices,
+                             const int32_t* last_page_len, int32_t batch, int32_t max_qo_tokens, int32_t page_size,
+                             int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim, int64_t* token_to_page,
+                             int64_t* token_to_cache, int32_t token_map_len, void* workspace,
+                             int64_t workspace_bytes, const HostIndices* host, void* stream) {
   if (batch < 0 || max_qo_tokens < 0 || token_map_len < 0 || !workspace) return MI_ERR_INVALID;
   if (!qo_indptr || !kv_indptr || !last_page_len || (batch > 0 && !kv_indices)) return MI_ERR_INVALID;
   if (token_map_len > 0 && (!token_to_page || !token_to_cache)) return MI_ERR_INVALID;
@@ -702,10 +728,46 @@ extern "C" int mi_prefill_plan(const int32_t* qo_indptr, const int32_t* kv_indpt
   m.t2c = token_to_cache;
   m.map_len = token_map_len;
   const int grid = 2 + (token_map_len + 1023) / 1024;
-  hipLaunchKernelGGL(prefill_plan_kernel, dim3(grid), dim3(1024), 0, (hipStream_t)stream, a, d, m);
+  if (host)
+    hipLaunchKernelGGL(prefill_plan_host_kernel, dim3(grid), dim3(1024), 0, (hipStream_t)stream, a, d, m, *host);
+  else
+    hipLaunchKernelGGL(prefill_plan_kernel, dim3(grid), dim3(1024), 0, (hipStream_t)stream, a, d, m);
   MI_CHECK_LAUNCH();
   return MI_OK;
 }
+
+}  // namespace mi
+
+extern "C" int mi_prefill_plan(const int32_t* qo_indptr, const int32_t* kv_indptr,
+                               const int32_t* kv_indices, const int32_t* last_page_len, int32_t batch,
+                               int32_t max_qo_tokens, int32_t page_size, int32_t num_qo_heads,
+                               int32_t num_kv_heads, int32_t head_dim, int64_t* token_to_page,
+                               int64_t* token_to_cache, int32_t token_map_len, void* workspace,
+                               int64_t workspace_bytes, void* stream) {
+  return mi::prefill_plan_impl(qo_indptr, kv_indptr, kv_indices, last_page_len, batch, max_qo_tokens, page_size,
+                               num_qo_heads, num_kv_heads, head_dim, token_to_page, token_to_cache, token_map_len,
+                               workspace, workspace_bytes, nullptr, stream);
+}
+
+extern "C" int mi_prefill_plan_host(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host,
+                                    const int32_t* kv_indices_host, const int32_t* last_page_len_host,
+                                    int32_t num_indices, int32_t* qo_indptr, int32_t* kv_indptr, int32_t* kv_indices,
+                                    int32_t* last_page_len, int32_t batch, int32_t max_qo_tokens, int32_t page_size,
+                                    int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim,
+                                    int64_t* token_to_page, int64_t* token_to_cache, int32_t token_map_len,
+                                    void* workspace, int64_t workspace_bytes, void* stream) {
+  if (batch < 0) return MI_ERR_INVALID;
+  const int32_t* const src[4] = {qo_indptr_host, kv_indptr_host, kv_indices_host, last_page_len_host};
+  int32_t* const dst[4] = {qo_indptr, kv_indptr, kv_indices, last_page_len};
+  const int32_t len[4] = {batch + 1, batch + 1, num_indices, batch};
+  mi::HostIndices m;
+  const int st = mi::host_indices(src, len, dst, 4, &m);
+  if (st != MI_OK) return st;
+  return mi::prefill_plan_impl(qo_indptr, kv_indptr, kv_indices, last_page_len, batch, max_qo_tokens, page_size,
+                               num_qo_heads, num_kv_heads, head_dim, token_to_page, token_to_cache, token_map_len,
+                               workspace, workspace_bytes, &m, stream);
+}
+
 
 namespace mi {
 

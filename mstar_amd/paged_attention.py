@@ -29,6 +29,7 @@ from __future__ import annotations
 
 import math
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -127,6 +128,23 @@ class _Staging:
             else:
                 outs.append(piece)
         return outs
+
+
+def _host_args(parts: list[torch.Tensor]) -> list[torch.Tensor] | None:
+    """The contiguous int32 CPU tensors of a plan whose indices travel in the
+    launch argument (``mi_*_plan_host``), or None: too many values, an empty
+    part, or a plan under graph capture (its staged copy is recorded there)."""
+    if sum(t.shape[0] for t in parts) > _lib.PLAN_HOST_ARGS or not all(t.dim() == 1 and t.shape[0] for t in parts):
+        return None
+    if torch.cuda.is_current_stream_capturing():
+        return None
+    return [t if t.dtype == torch.int32 and t.is_contiguous() else t.to(torch.int32).contiguous() for t in parts]
+
+
+def _carve(parts: list[torch.Tensor], device: torch.device) -> list[torch.Tensor]:
+    """Device int32 tensors of the parts' lengths, from one allocation."""
+    return list(torch.empty(sum(t.shape[0] for t in parts), dtype=torch.int32,
+                            device=device).split([t.shape[0] for t in parts]))
 
 
 def _as_device_int(t: torch.Tensor, dtype: torch.dtype, device: torch.device) -> torch.Tensor:
@@ -239,6 +257,7 @@ class PagedDecodeWrapper(_FusedRopeAppend):
         self.dtype = None
         self._workspace = workspace_buffer
         self._staging = _Staging()
+        self._indptr = self._retired = None
         self._n_req = 0
         if use_cuda_graph:
             assert batch_size is not None, "batch_size required for CUDA graph mode"
@@ -275,7 +294,11 @@ class PagedDecodeWrapper(_FusedRopeAppend):
         srcs = [paged_kv_indptr, paged_kv_indices, paged_kv_last_page_len]
         nv = self.enable_nvtx
         with trace_range(nv, "flashinfer.decode.metadata_h2d"):
-            if all(t.device.type == "cpu" for t in srcs):
+            on_cpu = all(t.is_cpu for t in srcs)
+            host = _host_args(srcs) if on_cpu else None
+            if host is not None:
+                indptr, indices, last = dests if self.use_cuda_graph else _carve(host, dev)
+            elif on_cpu:
                 srcs = [t.to(torch.int32) for t in srcs]
                 indptr, indices, last = self._staging.upload(srcs, dev, dests)
             else:
@@ -301,16 +324,16 @@ class PagedDecodeWrapper(_FusedRopeAppend):
             loc_out = self.kv_cache_locations
         # the split-KV plan; the write locations (the reference's kv_location_compute) come out of the same launch
         with trace_range(nv, "flashinfer.decode.plan_inner"):
-            _lib.check(
-                _lib.lib().mi_decode_plan(
-                    None, indptr.data_ptr(), indices.data_ptr(), last.data_ptr(), n_req, self.page_size,
-                    self.num_qo_heads, self.num_kv_heads, self.head_dim,
-                    loc_out.data_ptr() if loc_out is not None else None,
-                    self._workspace.data_ptr(), self._workspace.numel() * self._workspace.element_size(),
-                    _lib.stream_ptr(dev),
-                ),
-                "mi_decode_plan",
-            )
+            ws = self._workspace
+            args = (indptr.data_ptr(), indices.data_ptr(), last.data_ptr(), n_req, self.page_size, self.num_qo_heads,
+                    self.num_kv_heads, self.head_dim, loc_out.data_ptr() if loc_out is not None else None,
+                    ws.data_ptr(), ws.numel() * ws.element_size(), _lib.stream_ptr(dev))
+            if host is not None:
+                _lib.check(_lib.lib().mi_decode_plan_host(*[t.data_ptr() for t in host], host[1].shape[0], *args),
+                           "mi_decode_plan_host")
+            else:
+                _lib.check(_lib.lib().mi_decode_plan(None, *args), "mi_decode_plan")
+        self._retired = self._indptr  # a run() of the previous plan may still read its arrays on another stream
         self._indptr, self._indices, self._last = indptr, indices, last
         self._n_req = n_req
         self.dtype = dtype
@@ -414,6 +437,7 @@ class PagedPrefillWrapper(_FusedRopeAppend):
         self.causal = True
         self._workspace = workspace_buffer
         self._staging = _Staging()
+        self._indptr = self._retired = None
         # Side stream of run(): made here so that a run() under graph capture
         # only records the fork/join on it (creating a stream is not capturable).
         self._side = torch.cuda.Stream(device=self.device)
@@ -449,8 +473,8 @@ class PagedPrefillWrapper(_FusedRopeAppend):
         one device sync for device inputs (as the reference, ``:215``).
         """
         srcs = [qo_indptr, paged_kv_indptr, paged_kv_indices, paged_kv_last_page_len]
-        on_cpu = all(t.device.type == "cpu" for t in srcs)
-        total_tokens = int(qo_indptr[-1]) if on_cpu else int(qo_indptr[-1].item())
+        on_cpu = all(t.is_cpu for t in srcs)
+        total_tokens = int(qo_indptr.numpy()[-1]) if on_cpu else int(qo_indptr[-1].item())
         self._plan(qo_indptr, paged_kv_indptr, paged_kv_indices, paged_kv_last_page_len, total_tokens, causal, dtype)
 
     def plan_device(self, qo_indptr: torch.Tensor, paged_kv_indptr: torch.Tensor, paged_kv_indices: torch.Tensor,
@@ -468,7 +492,7 @@ class PagedPrefillWrapper(_FusedRopeAppend):
         self.dtype = dtype
         self.causal = bool(causal)
         srcs = [qo_indptr, paged_kv_indptr, paged_kv_indices, paged_kv_last_page_len]
-        on_cpu = all(t.device.type == "cpu" for t in srcs)
+        on_cpu = all(t.is_cpu for t in srcs)
         self._total_tokens = total_tokens
         if self.use_cuda_graph:
             if n_req != self.batch_size:  # captured launches bake the batch in
@@ -481,7 +505,10 @@ class PagedPrefillWrapper(_FusedRopeAppend):
                      self._paged_kv_last_page_len_buf]
         else:
             dests = [None] * 4
-        if on_cpu:
+        host = _host_args(srcs) if on_cpu else None
+        if host is not None:
+            qo, indptr, indices, last = dests if self.use_cuda_graph else _carve(host, dev)
+        elif on_cpu:
             qo, indptr, indices, last = self._staging.upload([t.to(torch.int32) for t in srcs], dev, dests)
         else:
             qo, indptr, indices, last = [_as_device_int(t, torch.int32, dev) for t in srcs]
@@ -497,15 +524,16 @@ class PagedPrefillWrapper(_FusedRopeAppend):
         batch = n_req
         max_tokens = self.max_total_tokens if self.use_cuda_graph else total_tokens
         ws_bytes = self._workspace.numel() * self._workspace.element_size()
-        _lib.check(
-            _lib.lib().mi_prefill_plan(
-                qo.data_ptr(), indptr.data_ptr(), indices.data_ptr(), last.data_ptr(), n_req, max_tokens,
+        args = (qo.data_ptr(), indptr.data_ptr(), indices.data_ptr(), last.data_ptr(), n_req, max_tokens,
                 self.page_size, self.num_qo_heads, self.num_kv_heads, self.head_dim,
                 self.token_to_page.data_ptr(), self.token_to_cache.data_ptr(), self.token_to_page.shape[0],
-                self._workspace.data_ptr(), ws_bytes, _lib.stream_ptr(dev),
-            ),
-            "mi_prefill_plan",
-        )
+                self._workspace.data_ptr(), ws_bytes, _lib.stream_ptr(dev))
+        if host is not None:
+            _lib.check(_lib.lib().mi_prefill_plan_host(*[t.data_ptr() for t in host], host[2].shape[0], *args),
+                       "mi_prefill_plan_host")
+        else:
+            _lib.check(_lib.lib().mi_prefill_plan(*args), "mi_prefill_plan")
+        self._retired = self._indptr  # a run() of the previous plan may still read its arrays on another stream
         self._qo, self._indptr, self._indices, self._last = qo, indptr, indices, last
         self._n_req = n_req
         self._plan_batch = batch
@@ -518,7 +546,7 @@ class PagedPrefillWrapper(_FusedRopeAppend):
             # a request of at most `short` (token, q-head) rows goes to the split-KV
             # decode kernel (mi_prefill_short), a longer one to the MFMA tiles
             short = _lib.lib().mi_prefill_short_rows(n_req, self.num_qo_heads, self.num_kv_heads, self.head_dim)
-            rows = torch.diff(qo_indptr.to(torch.int64)) * (self.num_qo_heads // self.num_kv_heads)
+            rows = np.diff(qo_indptr.numpy().astype(np.int64, copy=False)) * (self.num_qo_heads // self.num_kv_heads)
             self._run_short = bool(((rows > 0) & (rows <= short)).any())
             self._run_tiles = bool((rows > short).any())
         else:

@@ -1,0 +1,84 @@
+"""GPU: plans whose CPU index tensors travel in the launch argument.
+
+At the argument's limit of 800 values and one beyond it (the staged copy),
+plan() must leave the same arrays on the device, the same token map and write
+locations, and run() the same bits, as plan() over device tensors, which takes
+neither path; also in graph mode, where the arrays are static buffers.
+"""
+
+import pytest
+import torch
+
+from gpu_helpers import custom_batch, log, random_cache, workspace
+from mstar_amd import _lib
+from mstar_amd.paged_attention import FlashInferDecodeWrapper, FlashInferPrefillWrapper
+
+pytestmark = pytest.mark.gpu
+
+
+def _lens(batch, values, fixed, ps):
+    """Context lengths whose index arrays hold ``values`` values in all (``fixed`` beside the pages)."""
+    pages = values - fixed
+    per = pages // batch
+    return [ps * per - (7 * i) % ps for i in range(batch - 1)] + [ps * (pages - per * (batch - 1)) - 3]
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("extra", [-1, 0, 1])
+@pytest.mark.parametrize("batch", [1, 5, 200])
+def test_decode_plan_host(gpu, batch, extra, graph):
+    hq, hkv, d, ps = 8, 2, 128, 16
+    log(f"decode plan host batch={batch} extra={extra} graph={graph}")
+    lens = _lens(batch, _lib.PLAN_HOST_ARGS + extra, 2 * batch + 1, ps)
+    qo, indptr, indices, last = custom_batch(lens, ps, 1000, 3)
+    assert len(indptr) + len(indices) + len(last) == _lib.PLAN_HOST_ARGS + extra
+    cache = random_cache(1000, ps, hkv, d, 5).to(gpu)
+    q = torch.randn(batch, hq, d, device=gpu).to(torch.bfloat16)
+    got = []
+    for dev in ("cpu", gpu):
+        fixed = {"batch_size": batch, "max_num_pages": 1000, "use_cuda_graph": True} if graph else {}
+        w = FlashInferDecodeWrapper(workspace(gpu), hq, hkv, d, ps, device=gpu, **fixed)
+        w.plan(*(torch.as_tensor(x).to(dev) for x in (indptr, indices, last)))
+        out = w.run(q, cache)
+        got.append((out, w.kv_cache_locations, w._indptr, w._indices[: len(indices)], w._last))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    assert got[0][3].cpu().tolist() == indices.tolist()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("extra", [0, 1])
+@pytest.mark.parametrize("batch", [1, 40])
+def test_prefill_plan_host(gpu, batch, extra, graph):
+    hq, hkv, d, ps = 8, 2, 128, 16
+    log(f"prefill plan host batch={batch} extra={extra} graph={graph}")
+    lens = _lens(batch, _lib.PLAN_HOST_ARGS + extra, 3 * batch + 2, ps)
+    new = [min(n, 1 + 37 * (i % 3)) for i, n in enumerate(lens)]  # short-query and tiled requests
+    meta = custom_batch(lens, ps, 1000, 3, new_lens=new)
+    assert sum(len(x) for x in meta) == _lib.PLAN_HOST_ARGS + extra
+    cache = random_cache(1000, ps, hkv, d, 5).to(gpu)
+    q = torch.randn(sum(new), hq, d, device=gpu).to(torch.bfloat16)
+    got = []
+    for dev in ("cpu", gpu):
+        fixed = ({"batch_size": batch, "max_num_pages": 1000, "max_total_tokens": sum(new) + 5, "use_cuda_graph": True}
+                 if graph else {})
+        w = FlashInferPrefillWrapper(workspace(gpu), hq, hkv, d, ps, device=gpu, **fixed)
+        w.plan(*(torch.as_tensor(x).to(dev) for x in meta))
+        out = w.run(q, cache)
+        got.append((out, w.token_to_page, w.token_to_cache, w._qo, w._indptr, w._indices[: len(meta[2])], w._last))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
+def test_plan_host_leaves_the_caller_its_tensors(gpu):
+    """The indices are read before plan() returns: a caller may overwrite them at once."""
+    log("plan host: inputs overwritten after plan()")
+    hq, hkv, d, ps = 8, 2, 128, 16
+    qo, indptr, indices, last = custom_batch([100, 300], ps, 64, 3)
+    parts = [torch.as_tensor(x).clone() for x in (indptr, indices, last)]
+    w = FlashInferDecodeWrapper(workspace(gpu), hq, hkv, d, ps, device=gpu)
+    w.plan(*parts)
+    for t in parts:
+        t.fill_(-1)
+    torch.cuda.synchronize()
+    assert w._indices.cpu().tolist() == indices.tolist() and w._indptr.cpu().tolist() == indptr.tolist()
