@@ -353,6 +353,11 @@ int mi_prefill_tiles(const void* q, int32_t q_dtype, int64_t q_stride_token, int
  * ------------------------------------------------------------------------ */
 int mi_rope_positions(const int32_t* qo_indptr, const int32_t* position_id_start, int32_t batch,
                       int64_t* pos_ids, int32_t num_tokens, void* stream);
+/* The same with both arrays in host memory, carried by the launch argument:
+ * at most MI_PLAN_HOST_ARGS values (2 * batch + 1), MI_ERR_UNSUPPORTED beyond.
+ * The arrays are not read after the call returns. */
+int mi_rope_positions_host(const int32_t* qo_indptr_host, const int32_t* position_id_start_host, int32_t batch,
+                           int64_t* pos_ids, int32_t num_tokens, void* stream);
 int mi_rope_apply(void* q, int64_t q_stride_token, int64_t q_stride_head, int32_t num_qo_heads, void* k,
                   int64_t k_stride_token, int64_t k_stride_head, int32_t num_kv_heads, int32_t dtype,
                   int32_t head_dim, int32_t rotary_dim, const void* pos_ids, int32_t pos_dtype,

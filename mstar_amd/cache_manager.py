@@ -392,8 +392,7 @@ class BatchedCacheManager:
             n = int(meta[b]) if b else 0
             out = torch.empty(n, dtype=torch.long, device=self.device)
             if n:
-                dev = self._pack.upload(meta)
-                rope_positions(dev[: b + 1], dev[b + 1:], out, n)
+                self._expand_positions(meta, b, out, n)
             parts.append(out)
         self._plan_states[combined_label].pos_ids = parts[0] if len(parts) == 1 else torch.cat(parts)
 
@@ -505,9 +504,19 @@ class BatchedCacheManager:
             if n:
                 # the positions are expanded on the device from one small upload
                 with trace_range(nv, "cache.plan_rope.copy_pos_ids"):
-                    dev = self._pack.upload(meta)
-                    rope_positions(dev[: b + 1], dev[b + 1:], out, n)
+                    self._expand_positions(meta, b, out, n)
             ps.pos_ids = out
+
+    def _expand_positions(self, meta: np.ndarray, b: int, out: torch.Tensor, n: int) -> None:
+        """``out`` from ``[cumulative lengths (b + 1) | starts (b)]``: in the launch argument where they fit
+        (a captured launch would keep its values), else through one small upload."""
+        if meta.size <= _lib.PLAN_HOST_ARGS and not torch.cuda.is_current_stream_capturing():
+            base = meta.ctypes.data
+            _lib.check(_lib.lib().mi_rope_positions_host(base, base + 4 * (b + 1), b, out.data_ptr(), n,
+                                                         _lib.stream_ptr(out.device)), "mi_rope_positions_host")
+            return
+        dev = self._pack.upload(meta)
+        rope_positions(dev[: b + 1], dev[b + 1:], out, n)
 
     def apply_rope(self, q: torch.Tensor, k: torch.Tensor, rotary_dim: int | None = None, interleave: bool = False,
                    rope_scale: float = 1, rope_theta: float = 10000.0, rope_dtype=None, **kwargs):
