@@ -43,6 +43,16 @@ __all__ = [
 ]
 
 _MAX_GROUP = 16  # q heads per kv head handled by one MFMA tile
+# Ragged batches of up to _SERIAL_REQUESTS requests run their two parts one
+# after the other on one stream: the events of a fork and join cost the host
+# more than the overlap hides (us a layer, side stream -> in turn: one 512-token
+# chunk and 3 decodes 77 -> 57, a 2048-token chunk and 7 decodes of up to 32k
+# tokens 193 -> 176, two chunks and 14 decodes 239 -> 237; 8 chunks and 120
+# decodes 601 -> 635, so those fork).  A captured graph has no host in it, but
+# launches both parts whatever it is replayed on: in turn only where the tiles
+# are few (two 50-token suffixes, 8 layers: 247 -> 221; a 512-token chunk and 3
+# decodes 55 -> 58).
+_SERIAL_REQUESTS, _SERIAL_GRAPH_ROWS = 16, 8192
 
 
 def _check_heads(num_qo_heads: int, num_kv_heads: int, head_dim: int, page_size: int) -> None:
@@ -536,6 +546,8 @@ class PagedPrefillWrapper(_FusedRopeAppend):
         self._retired = self._indptr  # a run() of the previous plan may still read its arrays on another stream
         self._qo, self._indptr, self._indices, self._last = qo, indptr, indices, last
         self._n_req = n_req
+        self._serial = n_req <= _SERIAL_REQUESTS and (
+            not self.use_cuda_graph or self.max_total_tokens * self.num_qo_heads <= _SERIAL_GRAPH_ROWS)
         self._plan_batch = batch
         self._plan_max_tokens = max_tokens
         # Which of run()'s two launches has work: known on the host for CPU
@@ -576,10 +588,14 @@ class PagedPrefillWrapper(_FusedRopeAppend):
                 self._plan_max_tokens, self.num_qo_heads, 1 if self.causal else 0, 1.0 / math.sqrt(self.head_dim),
                 self._workspace.data_ptr(), ws_bytes, out.data_ptr(), os_[0], os_[1], None]
         # The MFMA tiles (long-query requests) and the split-KV decode of the
-        # short-query requests write disjoint rows: run the HBM-bound decode
-        # on a side stream so it overlaps the compute-bound tiles.
+        # short-query requests write disjoint rows: where the batch can hold much
+        # of both, the HBM-bound decode runs on a side stream, so that it overlaps
+        # the compute-bound tiles.
         main = torch.cuda.current_stream(q.device)
-        if self._run_tiles and self._run_short:
+        if self._run_tiles and self._run_short and self._serial:
+            args[-1] = main.cuda_stream
+            _lib.check(_lib.lib().mi_prefill_run(*args), "mi_prefill_run")
+        elif self._run_tiles and self._run_short:
             side = self._side
             side.wait_stream(main)
             args[-1] = main.cuda_stream
