@@ -97,6 +97,10 @@ SIGNATURES = {
         ctypes.c_int,
         [_P, _P, _P, _I32, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _P, _P, _I64, _P],
     ),
+    "mi_decode_plan_pinned": (
+        ctypes.c_int,
+        [_P, _I32, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _P, _P, _I64, _P],
+    ),
     "mi_decode_run": (
         ctypes.c_int,
         [_P, _I32, _I64, _I64, ctypes.POINTER(MiPagedKV), _P, _P, _P, _P, _I32, _I32, _I32, _F32,
@@ -267,6 +271,7 @@ def _event_create(device: torch.device) -> int:
     return ev.value
 
 
+PLAN_PINNED_BATCH = 1024  # MI_PLAN_PINNED_BATCH
 PLAN_HOST_ARGS = 800  # MI_PLAN_HOST_ARGS: int32 values of host index arrays a plan call passes as a kernel argument
 PACK_HOST_META = 768  # MI_PACK_HOST_META: int32 values of step metadata always passed as a kernel argument
 PACK_HOST_META_MAX = 4096  # MI_PACK_HOST_META_MAX: up to this many when the step fits the argument's compact form
@@ -317,6 +322,62 @@ class PinnedUploader:
             if rc != 0:
                 raise RuntimeError(f"hipEventRecord failed with HIP error {rc}")
         return dev if n == dev.shape[0] else dev[:n]
+
+
+class PinnedRing:
+    """Pinned host rows that a launch reads by itself (``mi_decode_plan_pinned``).
+
+    ``SLOTS`` rows of ``VALUES`` int32 each are used in turn; an event recorded
+    behind the launch guards a row until its next use, so a caller waits only
+    for the launch ``SLOTS`` calls ago.  Rows are never freed while a launch may
+    read them: use the per-device instance from :func:`pinned_ring`, which lives
+    for the process.
+    """
+
+    SLOTS, VALUES = 8, 16384
+
+    def __init__(self, device: torch.device):
+        self.device = torch.device(device)
+        self._mem = torch.empty(self.SLOTS, self.VALUES, dtype=torch.int32, pin_memory=True)
+        self._rows = self._mem.numpy()
+        self._ptrs = [self._mem[i].data_ptr() for i in range(self.SLOTS)]
+        self._events: list = [None] * self.SLOTS
+        self._next = 0
+        self._lock = threading.Lock()
+
+    def launch(self, parts, stream: int, fn) -> None:
+        """Write ``parts`` (CPU tensors) one after the other and call ``fn(address)``, which launches on ``stream``."""
+        _, record, sync = _events_api()
+        with self._lock:
+            i = self._next
+            self._next = (i + 1) % self.SLOTS
+            ev = self._events[i]
+            if ev is None:
+                ev = self._events[i] = _event_create(self.device)
+            elif (rc := sync(ev)) != 0:
+                raise RuntimeError(f"hipEventSynchronize failed with HIP error {rc}")
+            row, at = self._rows[i], 0
+            for t in parts:
+                row[at:at + t.shape[0]] = t.numpy()
+                at += t.shape[0]
+            fn(self._ptrs[i])
+            rc = record(ev, stream)
+            if rc != 0:
+                raise RuntimeError(f"hipEventRecord failed with HIP error {rc}")
+
+
+_rings: dict = {}
+
+
+def pinned_ring(device: torch.device) -> PinnedRing:
+    """The process-wide :class:`PinnedRing` of ``device``."""
+    r = _rings.get(device)
+    if r is None:
+        with _uploaders_lock:
+            r = _rings.get(device)
+            if r is None:
+                r = _rings[device] = PinnedRing(device)
+    return r
 
 
 _uploaders: dict = {}

@@ -18,6 +18,18 @@ inline int device_cu_count() {
   return cached[dev];
 }
 
+// Memory a kernel may touch: HIP device memory, or host memory that HIP
+// allocated pinned (reachable over the bus at the same address).  Pageable
+// host memory is not.
+inline bool device_reachable(const void* ptr) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, ptr) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type == hipMemoryTypeDevice || a.type == hipMemoryTypeHost || a.type == hipMemoryTypeManaged;
+}
+
 // Workspace layout of a split-KV plan (decode kernel + merge).
 struct SplitLayout {
   int64_t hdr, chunk_indptr, work, lse, opart, total;

@@ -6,6 +6,7 @@
 // page is moved in 16-byte vectors by a grid-stride loop.  Pages whose ids
 // fall outside [0, max_pages) are skipped.
 #include "mi_common.h"
+#include "mi_internal.h"
 
 namespace mi {
 
@@ -186,18 +187,6 @@ __global__ __launch_bounds__(256) void kv_segments_kernel(SegParams p) {
       }
     }
   }
-}
-
-// Memory a kernel may touch: HIP device memory, or host memory that HIP
-// allocated pinned (reachable over the bus at the same address).  Pageable
-// host memory is not.
-static bool device_reachable(const void* ptr) {
-  hipPointerAttribute_t a;
-  if (hipPointerGetAttributes(&a, ptr) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
-  return a.type == hipMemoryTypeDevice || a.type == hipMemoryTypeHost || a.type == hipMemoryTypeManaged;
 }
 
 static int seg_pool_check(const mi_kv_pool* p, int32_t layer_end) {

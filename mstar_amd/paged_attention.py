@@ -151,6 +151,12 @@ def _host_args(parts: list[torch.Tensor]) -> list[torch.Tensor] | None:
     return [t if t.dtype == torch.int32 and t.is_contiguous() else t.to(torch.int32).contiguous() for t in parts]
 
 
+def _pinned_args(parts: list[torch.Tensor], n_req: int) -> bool:
+    """Whether a plan launch can read these CPU tensors from pinned memory (``mi_decode_plan_pinned``)."""
+    return (sum(t.shape[0] for t in parts) <= _lib.PinnedRing.VALUES and 0 < n_req <= _lib.PLAN_PINNED_BATCH
+            and all(t.dim() == 1 and t.shape[0] for t in parts) and not torch.cuda.is_current_stream_capturing())
+
+
 def _carve(parts: list[torch.Tensor], device: torch.device) -> list[torch.Tensor]:
     """Device int32 tensors of the parts' lengths, from one allocation."""
     return list(torch.empty(sum(t.shape[0] for t in parts), dtype=torch.int32,
@@ -306,8 +312,9 @@ class PagedDecodeWrapper(_FusedRopeAppend):
         with trace_range(nv, "flashinfer.decode.metadata_h2d"):
             on_cpu = all(t.is_cpu for t in srcs)
             host = _host_args(srcs) if on_cpu else None
-            if host is not None:
-                indptr, indices, last = dests if self.use_cuda_graph else _carve(host, dev)
+            pinned = on_cpu and host is None and _pinned_args(srcs, n_req)
+            if host is not None or pinned:
+                indptr, indices, last = dests if self.use_cuda_graph else _carve(srcs, dev)
             elif on_cpu:
                 srcs = [t.to(torch.int32) for t in srcs]
                 indptr, indices, last = self._staging.upload(srcs, dev, dests)
@@ -341,6 +348,11 @@ class PagedDecodeWrapper(_FusedRopeAppend):
             if host is not None:
                 _lib.check(_lib.lib().mi_decode_plan_host(*[t.data_ptr() for t in host], host[1].shape[0], *args),
                            "mi_decode_plan_host")
+            elif pinned:
+                n_idx = paged_kv_indices.shape[0]
+                _lib.pinned_ring(dev).launch(
+                    (paged_kv_indptr, paged_kv_last_page_len, paged_kv_indices), args[-1],
+                    lambda at: _lib.check(_lib.lib().mi_decode_plan_pinned(at, n_idx, *args), "mi_decode_plan_pinned"))
             else:
                 _lib.check(_lib.lib().mi_decode_plan(None, *args), "mi_decode_plan")
         self._retired = self._indptr  # a run() of the previous plan may still read its arrays on another stream

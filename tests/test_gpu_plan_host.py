@@ -82,3 +82,31 @@ def test_plan_host_leaves_the_caller_its_tensors(gpu):
         t.fill_(-1)
     torch.cuda.synchronize()
     assert w._indices.cpu().tolist() == indices.tolist() and w._indptr.cpu().tolist() == indptr.tolist()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("batch,values", [(1, 801), (64, 5000), (1024, 16384), (1024, 16385), (1025, 16384)])
+def test_decode_plan_pinned(gpu, batch, values, graph):
+    """Index arrays in pinned memory up to its 16384 values and 1024 requests, the staged copy
+    beyond, against device tensors; more plans in flight than the ring has rows."""
+    hq, hkv, d, ps = 8, 2, 128, 16
+    log(f"decode plan pinned batch={batch} values={values} graph={graph}")
+    lens = _lens(batch, values, 2 * batch + 1, ps)
+    qo, indptr, indices, last = custom_batch(lens, ps, 17000, 3)
+    assert len(indptr) + len(indices) + len(last) == values
+    cache = torch.randn(17000, 2, ps, hkv, d, device=gpu, dtype=torch.bfloat16)
+    q = torch.randn(batch, hq, d, device=gpu).to(torch.bfloat16)
+    got = []
+    for dev, dtype in (("cpu", torch.int64), (gpu, torch.int32)):
+        fixed = {"batch_size": batch, "max_num_pages": 17000, "use_cuda_graph": True} if graph else {}
+        w = FlashInferDecodeWrapper(workspace(gpu), hq, hkv, d, ps, device=gpu, **fixed)
+        other = [torch.as_tensor(x).to(dev, dtype) for x in (indptr, indices[::-1].copy(), last)]
+        parts = [torch.as_tensor(x).to(dev, dtype) for x in (indptr, indices, last)]
+        for _ in range(2 * _lib.PinnedRing.SLOTS):
+            w.plan(*other)
+            w.plan(*parts)
+        out = w.run(q, cache)
+        got.append((out, w.kv_cache_locations, w._indptr, w._indices[: len(indices)], w._last))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    assert got[0][3].cpu().tolist() == indices.tolist()
