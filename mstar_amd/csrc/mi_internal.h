@@ -184,7 +184,7 @@ int decode_run_impl(const void* q, int32_t q_dtype, int64_t q_stride_token, int6
                     int32_t num_qo_heads, int32_t causal, float sm_scale, void* workspace,
                     int64_t workspace_bytes, int64_t ws_offset, void* out,
                     int64_t out_stride_token, int64_t out_stride_head, int phases, hipStream_t stream,
-                    bool ragged_pair = false);
+                    bool ragged_pair = false, DecodeParams* merge_args = nullptr);
 
 // Wavefront scans and reductions on the VALU's cross-lane paths: one row_shr
 // per power of two within a 16-lane row, then two row broadcasts.  (__shfl

@@ -34,6 +34,7 @@
 // per-head scales multiply the scores and the output.
 #include "mi_prefill_kernel.h"
 #include "mi_prefill_rs.h"
+#include "mi_merge.h"
 
 namespace mi {
 constexpr int kShortRows = kShortRowsMax;  // qo_len * group <= 16 -> decode kernel (8 on a paired plan)
@@ -568,13 +569,13 @@ static int launch_prefill(const PrefillParams& pp, int head_dim, int grid, hipSt
 // tiles took 63 and 84 us of kernel against 44 + 8.)
 constexpr int kPfMergeThreads = 512;
 template <typename MT, int D>
-__global__ __launch_bounds__(kPfMergeThreads) void prefill_merge_kernel(PrefillParams p) {
-  constexpr int VW = D / 16, NV = D / 64, ROWS = pf_rows(D), NG = ROWS / 16, U = D > 128 ? 4 : 8, WAVES = kPfMergeThreads / 64;
+MI_DEVICE void prefill_merge_body(const PrefillParams& p, int first_wave, int waves) {
+  constexpr int VW = D / 16, NV = D / 64, ROWS = pf_rows(D), NG = ROWS / 16, U = D > 128 ? 4 : 8;
   constexpr float kNegInf = -__builtin_inff();
   const int nkv = p.num_kv_heads, G = p.group;
   const int lane = lane_id(), col = lane & 15, grp = lane >> 4;
   const int total = p.hdr[kPfSplitTiles] * nkv * NG * 4;
-  for (int w = uniform((int)blockIdx.x * WAVES + ((int)threadIdx.x >> 6)); w < total; w += (int)gridDim.x * WAVES) {
+  for (int w = uniform(first_wave + ((int)threadIdx.x >> 6)); w < total; w += waves) {
     const int part = w & 3, rgi = (w >> 2) % NG, th = (w >> 2) / NG;
     const int h = th % nkv;
     const int4 st = p.split_tiles[th / nkv];
@@ -634,6 +635,37 @@ __global__ __launch_bounds__(kPfMergeThreads) void prefill_merge_kernel(PrefillP
     for (int i = 0; i < NV; ++i)
       *(uint2*)(orow + 16 * (NV * part + i) + 4 * grp) =
           make_uint2(MT::pack2(acc[i].x * inv, acc[i].y * inv), MT::pack2(acc[i].z * inv, acc[i].w * inv));
+  }
+}
+
+template <typename MT, int D>
+__global__ __launch_bounds__(kPfMergeThreads) void prefill_merge_kernel(PrefillParams p) {
+  constexpr int WAVES = kPfMergeThreads / 64;
+  prefill_merge_body<MT, D>(p, (int)blockIdx.x * WAVES, (int)gridDim.x * WAVES);
+}
+
+// Both merges of a call that runs both parts in turn: workgroups below
+// batch * nkv merge the short-query requests' split-KV items, the others the
+// split tiles (8 wavefronts a CU at most, as in the launch of their own).  A
+// dependent launch costs 4 us, whatever it does: two captured 50-token suffixes
+// over 8 layers take 205 us against 221 with a launch each.  A batch whose
+// decode plan pairs kv-heads keeps two launches.
+template <typename MT, int D, int RUN>
+__global__ __launch_bounds__(256) void both_merges_kernel(DecodeParams d, int32_t batch, PrefillParams p) {
+  const int shorts = batch * d.num_kv_heads;
+  if ((int)blockIdx.x < shorts)
+    merge_body<MT, D, RUN>(d, batch, (int)blockIdx.x);
+  else
+    prefill_merge_body<MT, D>(p, ((int)blockIdx.x - shorts) * 4, ((int)gridDim.x - shorts) * 4);
+}
+
+template <typename MT, bool FP8>
+static void launch_both_merges(const DecodeParams& d, int batch, const PrefillParams& p, int head_dim, int grid,
+                               hipStream_t stream) {
+  switch (head_dim) {
+    case 64: hipLaunchKernelGGL((both_merges_kernel<MT, 64, lane_run(64, FP8 ? 1 : 2)>), dim3(grid), dim3(256), 0, stream, d, batch, p); break;
+    case 128: hipLaunchKernelGGL((both_merges_kernel<MT, 128, lane_run(128, FP8 ? 1 : 2)>), dim3(grid), dim3(256), 0, stream, d, batch, p); break;
+    default: hipLaunchKernelGGL((both_merges_kernel<MT, 256, lane_run(256, FP8 ? 1 : 2)>), dim3(grid), dim3(256), 0, stream, d, batch, p); break;
   }
 }
 
@@ -806,10 +838,16 @@ static int prefill_run_impl(const void* q, int32_t q_dtype, int64_t q_stride_tok
   if (workspace_bytes < L.split) return MI_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
   int st = MI_OK;
+  const PfSplitLayout P = pf_split_of(L, batch, G, nkv, D, workspace_bytes);
+  // both parts in one call: one launch merges both (both_merges_kernel)
+  const bool both = phases == (kPhaseShort | kPhaseTiles) && P.parts > 0 && q_dtype != MI_F32 &&
+                    !pair_heads(nullptr, batch, nkv, G, D, true);
+  DecodeParams dmerge{};
   if (phases & kPhaseShort) {
     st = decode_run_impl(q, q_dtype, q_stride_token, q_stride_head, kv, qo_indptr, kv_indptr, kv_indices,
                          last_page_len, batch, num_qo_heads, causal, sm_scale, workspace, workspace_bytes,
-                         L.split, out, out_stride_token, out_stride_head, kPhaseAttend | kPhaseMerge, s, true);
+                         L.split, out, out_stride_token, out_stride_head, kPhaseAttend | (both ? 0 : kPhaseMerge), s,
+                         true, &dmerge);
     if (st != MI_OK) return st;
   }
   if (!(phases & kPhaseTiles)) return MI_OK;
@@ -862,7 +900,6 @@ static int prefill_run_impl(const void* q, int32_t q_dtype, int64_t q_stride_tok
   pp.tiles = (const int2*)(ws + L.tiles);
   pp.order = (const int32_t*)(ws + L.order);
   pp.ctr = (int32_t*)((uint8_t*)workspace + L.ctr);
-  const PfSplitLayout P = pf_split_of(L, batch, G, nkv, D, workspace_bytes);
   pp.pieces = (const int4*)(ws + P.pieces);
   pp.split_tiles = (const int4*)(ws + P.split_tiles);
   pp.part_lse = (float*)((uint8_t*)workspace + P.lse);
@@ -887,7 +924,14 @@ static int prefill_run_impl(const void* q, int32_t q_dtype, int64_t q_stride_tok
   if (st != MI_OK) return st;
   // which tiles are split is the device's decision: the merge is launched
   // wherever a split is possible, and exits at once without one (4 us)
-  if (P.parts > 0) {
+  if (both) {
+    const int64_t waves = (int64_t)L.max_tiles * nkv * (pf_rows(D) / 16) * 4;
+    const int grid2 = batch * nkv + (int)(waves < 8LL * ncu ? (waves + 3) / 4 : 2LL * ncu);
+    if (q_dtype == MI_BF16)
+      fp8 ? launch_both_merges<BF16, true>(dmerge, batch, pp, D, grid2, s) : launch_both_merges<BF16, false>(dmerge, batch, pp, D, grid2, s);
+    else
+      fp8 ? launch_both_merges<F16, true>(dmerge, batch, pp, D, grid2, s) : launch_both_merges<F16, false>(dmerge, batch, pp, D, grid2, s);
+  } else if (P.parts > 0) {
     const int64_t waves = (int64_t)L.max_tiles * nkv * (pf_rows(D) / 16) * 4, per = kPfMergeThreads / 64;
     const int mgrid = (int)(waves < ncu * per ? (waves + per - 1) / per : ncu);
     if (q_dtype == MI_BF16) launch_prefill_merge<BF16>(pp, D, mgrid, s);

@@ -97,3 +97,40 @@ def test_split_tiles_keep_non_finite_rows(gpu, hq, hkv, d):
     out, _ = _run(gpu, ROOMY, (hq, hkv, d), ps, meta, True, torch.bfloat16, cache, q, (None, None))
     first = at - (kv - new)
     assert torch.equal(out[:first], clean[:first]) and bool(out[first:].isnan().all())
+
+
+@pytest.mark.parametrize("heads,dtype,fp8,short,long", [
+    ((28, 4, 128), torch.bfloat16, False, [20000, 40, 9000], [(3000, 100)]),
+    ((28, 4, 128), torch.float16, True, [20000], [(3000, 33), (40, 40)]),     # one tile cut, one whole
+    ((8, 1, 256), torch.bfloat16, False, [9000, 1], [(850, 50), (1001, 3)]),  # 24 rows: the smallest tile
+    ((16, 2, 256), torch.bfloat16, True, [5000], [(1500, 77)]),
+    ((16, 4, 64), torch.float16, False, [9000, 300], [(3000, 90)]),
+    ((16, 4, 64), torch.bfloat16, True, [16], [(16, 16)]),                    # nothing to merge on either side
+])
+def test_one_merge_launch_for_both_parts(gpu, heads, dtype, fp8, short, long):
+    """Both parts in one call merge in one launch: the rows' arithmetic is that of
+    a merge launch each (the two-stream route), so the results are equal bit for bit."""
+    hq, hkv, d = heads
+    log(f"one merge launch {heads} {dtype} fp8={fp8} short={short} long={long}")
+    ps, kv_lens = 16, [n for n, _ in long] + short
+    meta = custom_batch(kv_lens, ps, int(sum(-(-np.array(kv_lens) // ps))) + 4, 3,
+                        new_lens=[n for _, n in long] + [1] * len(short))
+    pool = int(meta[2].max()) + 1
+    cache = random_cache(pool, ps, hkv, d, 5).to(gpu)
+    scales = (None, None)
+    if fp8:
+        cache, scales = cache.to(torch.float8_e4m3fn), (torch.full((hkv,), 0.5, device=gpu),) * 2
+    elif cache.dtype != dtype:
+        cache = cache.to(dtype)
+    q = torch.randn(int(meta[0][-1]), hq, d, generator=torch.Generator().manual_seed(6)).to(dtype).to(gpu)
+    w = FlashInferPrefillWrapper(workspace(gpu, ROOMY), *heads, ps, device=gpu)
+    w.plan(*(torch.as_tensor(x) for x in meta), causal=True, dtype=dtype)
+    outs = []
+    for serial in (True, False):
+        w._serial = serial
+        out = torch.full_like(q, float("nan"))
+        outs.append(w.run(q, cache, *scales, out=out))
+        torch.cuda.synchronize()
+    assert bool(outs[0].isfinite().all())
+    assert torch.equal(outs[0], outs[1])
+    assert (_hdr(w._workspace)[2] > _hdr(w._workspace)[0]) == (max(n for n, _ in long) > 16)
