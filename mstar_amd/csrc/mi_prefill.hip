@@ -5,12 +5,14 @@
 // plan:  one launch (prefill_plan_kernel): the token map (the per-new-token
 //        (page, slot) of flashinfer_utils.py:211-256), the tiles of every
 //        long-query request, costed and put as (kv-head, tile) units, or
-//        pieces of them, into 8 per-XCD queues (pf_choose), and, for the short-query requests
-//        (qo_len * group <= 16, e.g. the decode rows of a mixed batch), a
-//        split-KV plan for the decode kernel in the same workspace.
+//        pieces of them, into 8 per-XCD queues (pf_choose), and, for the
+//        short-query requests (qo_len * group <= 16, e.g. the decode rows of
+//        a mixed batch), a split-KV plan for the decode kernel in the same
+//        workspace.
 // run:   mi_prefill_short (decode kernel + merge for the short-query
 //        requests) and mi_prefill_tiles (prefill_kernel, and the merge of
-//        tiles that the plan has cut into key pieces).
+//        tiles that the plan has cut into key pieces); mi_prefill_run does
+//        both in turn, with one launch for the two merges.
 //
 // prefill_kernel (persistent, one workgroup per CU): a unit is a tile of
 // 256 (query token, q-head) rows of one request and kv-head -- GQA rows
@@ -203,10 +205,11 @@ static PfSplitCosts pf_split_costs(int head_dim) {
 // units per CU a queue of one request's long units ends long after the others
 // (4 chunks of 512-2048 tokens, 32 q / 4 kv heads, fp8 cache: 437 us from the
 // local queues, 320 us dealt).  Where the local queues are as even as a deal
-// they stay: 8 x 2048 tokens at head_dim 256 1262 us local, 1286 us dealt.  Each candidate is priced, one wavefront each, by the bounds that
-// any schedule of units u_1 >= u_2 >= ... on m workgroups obeys: their mean
-// load, and (k + 1) u_{km + 1} for each k (of the km + 1 longest, k + 1 share
-// a workgroup).  Heaviest-first queues come close to the larger of the two.
+// they stay: 8 x 2048 tokens at head_dim 256 1262 us local, 1286 us dealt.
+// Each candidate is priced, one wavefront each, by the bounds that any schedule
+// of units u_1 >= u_2 >= ... on m workgroups obeys: their mean load, and
+// (k + 1) u_{km + 1} for each k (of the km + 1 longest, k + 1 share a
+// workgroup).  Heaviest-first queues come close to the larger of the two.
 // The bounds are taken over all workgroups, and for kPfLocal also over each
 // queue's units on the queue's eighth of them.
 constexpr int kPfLocal = 0, kPfWhole = 0x7fffffff;
