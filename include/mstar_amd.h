@@ -328,6 +328,13 @@ int mi_decode_plan_pinned(const int32_t* indices_pinned, int32_t num_indices, in
                           int32_t* kv_indices, int32_t* last_page_len, int32_t batch, int32_t page_size,
                           int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim, int64_t* kv_locations,
                           void* workspace, int64_t workspace_bytes, void* stream);
+/* mi_prefill_plan likewise: [qo_indptr (batch + 1) | kv_indptr (batch + 1) |
+ * last_page_len (batch) | kv_indices (num_indices)] in pinned host memory. */
+int mi_prefill_plan_pinned(const int32_t* indices_pinned, int32_t num_indices, int32_t* qo_indptr,
+                           int32_t* kv_indptr, int32_t* kv_indices, int32_t* last_page_len, int32_t batch,
+                           int32_t max_qo_tokens, int32_t page_size, int32_t num_qo_heads, int32_t num_kv_heads,
+                           int32_t head_dim, int64_t* token_to_page, int64_t* token_to_cache,
+                           int32_t token_map_len, void* workspace, int64_t workspace_bytes, void* stream);
 int mi_prefill_run(const void* q, int32_t q_dtype, int64_t q_stride_token, int64_t q_stride_head,
                    const mi_paged_kv* kv, const int32_t* qo_indptr, const int32_t* kv_indptr,
                    const int32_t* kv_indices, const int32_t* last_page_len, int32_t batch,

@@ -135,6 +135,10 @@ SIGNATURES = {
         ctypes.c_int,
         [_P, _P, _P, _P, _I32, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _P, _P, _I32, _P, _I64, _P],
     ),
+    "mi_prefill_plan_pinned": (
+        ctypes.c_int,
+        [_P, _I32, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _P, _P, _I32, _P, _I64, _P],
+    ),
     "mi_prefill_run": (
         ctypes.c_int,
         [_P, _I32, _I64, _I64, ctypes.POINTER(MiPagedKV), _P, _P, _P, _P, _I32, _I32, _I32, _I32, _F32,
@@ -325,7 +329,7 @@ class PinnedUploader:
 
 
 class PinnedRing:
-    """Pinned host rows that a launch reads by itself (``mi_decode_plan_pinned``).
+    """Pinned host rows that a launch reads by itself (``mi_*_plan_pinned``).
 
     ``SLOTS`` rows of ``VALUES`` int32 each are used in turn; an event recorded
     behind the launch guards a row until its next use, so a caller waits only

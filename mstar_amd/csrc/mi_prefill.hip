@@ -525,12 +525,9 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(PfPlanArgs a, PlanPa
   }
 }
 
-// The index arrays in the argument: every workgroup plans from its own copy in
-// LDS, workgroup 0 also writes the device arrays.
-__global__ __launch_bounds__(1024) void prefill_plan_host_kernel(PfPlanArgs a, PlanParams d, TokenMapArgs m, HostIndices h) {
-  __shared__ int32_t s_idx[MI_PLAN_HOST_ARGS];
-  host_indices_copy(h, s_idx, blockIdx.x == 0);
-  const int32_t *qo = s_idx, *kvp = s_idx + h.end[0], *idx = s_idx + h.end[1], *last = s_idx + h.end[2];
+// One workgroup's part of the plan, from index arrays of its own.
+__device__ inline void plan_part(PfPlanArgs& a, PlanParams& d, TokenMapArgs& m, const int32_t* qo, const int32_t* kvp,
+                                 const int32_t* idx, const int32_t* last) {
   if (blockIdx.x == 0) {
     a.qo_indptr = qo;
     a.kv_indptr = kvp;
@@ -549,6 +546,49 @@ __global__ __launch_bounds__(1024) void prefill_plan_host_kernel(PfPlanArgs a, P
     m.last_page_len = last;
     token_map_body(m, ((int)blockIdx.x - 2) * 1024 + (int)threadIdx.x);
   }
+}
+
+// The index arrays in the argument: every workgroup plans from its own copy in
+// LDS, workgroup 0 also writes the device arrays.
+__global__ __launch_bounds__(1024) void prefill_plan_host_kernel(PfPlanArgs a, PlanParams d, TokenMapArgs m, HostIndices h) {
+  __shared__ int32_t s_idx[MI_PLAN_HOST_ARGS];
+  host_indices_copy(h, s_idx, blockIdx.x == 0);
+  plan_part(a, d, m, s_idx, s_idx + h.end[0], s_idx + h.end[1], s_idx + h.end[2]);
+}
+
+// The index arrays in pinned host memory, for plans that the argument cannot
+// hold: every workgroup that plans reads the per-request ones over the bus into
+// LDS, workgroup 0 also writes their device copies, the token map reads the
+// pages of its tokens over the bus, and the last workgroups copy the page list.
+// The staged copy (a copy on a side stream, events, and in graph mode four
+// device copies) took the host 65 us a plan: 6 chunks and 17 decodes of up to
+// 5.7k tokens, a layer launched eagerly, 205 -> 139 us a pass; 4 chunks over up
+// to 8k cached tokens with an fp8 cache, bound by their tiles, 322 -> 317.
+struct PfPinned {
+  const int32_t* src;  // [qo_indptr | kv_indptr | last_page_len | kv_indices]
+  int32_t num_indices, copy_blocks;
+  int32_t *qo_indptr, *kv_indptr, *last_page_len, *kv_indices;
+};
+__global__ __launch_bounds__(1024) void prefill_plan_pinned_kernel(PfPlanArgs a, PlanParams d, TokenMapArgs m, PfPinned h) {
+  __shared__ int32_t s_idx[3 * MI_PLAN_PINNED_BATCH + 2];
+  const int b = a.batch, per_request = 3 * b + 2;
+  const int32_t* idx = h.src + per_request;
+  const int copy = (int)blockIdx.x - ((int)gridDim.x - h.copy_blocks);
+  if (copy >= 0) {
+    for (int i = copy * 1024 + (int)threadIdx.x; i < h.num_indices; i += h.copy_blocks * 1024) h.kv_indices[i] = idx[i];
+    return;
+  }
+  for (int i = (int)threadIdx.x; i < per_request; i += 1024) {
+    const int32_t v = h.src[i];
+    s_idx[i] = v;
+    if (blockIdx.x == 0) {
+      if (i <= b) h.qo_indptr[i] = v;
+      else if (i <= 2 * b + 1) h.kv_indptr[i - b - 1] = v;
+      else h.last_page_len[i - 2 * b - 2] = v;
+    }
+  }
+  __syncthreads();
+  plan_part(a, d, m, s_idx, s_idx + b + 1, idx, s_idx + 2 * b + 2);
 }
 
 template <typename MT, bool FP8>
@@ -704,12 +744,12 @@ extern "C" int32_t mi_prefill_short_rows(int32_t batch, int32_t num_qo_heads, in
 
 namespace mi {
 
-// host: the index arrays in the launch argument, or NULL
+// host / pinned: the index arrays in the launch argument or in pinned memory (both NULL: the device arrays)
 static int prefill_plan_impl(const int32_t* qo_indptr, const int32_t* kv_indptr, const int32_t* kv_indices,
                              const int32_t* last_page_len, int32_t batch, int32_t max_qo_tokens, int32_t page_size,
                              int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim, int64_t* token_to_page,
                              int64_t* token_to_cache, int32_t token_map_len, void* workspace,
-                             int64_t workspace_bytes, const HostIndices* host, void* stream) {
+                             int64_t workspace_bytes, const HostIndices* host, PfPinned* pinned, void* stream) {
   if (batch < 0 || max_qo_tokens < 0 || token_map_len < 0 || !workspace) return MI_ERR_INVALID;
   if (!qo_indptr || !kv_indptr || !last_page_len || (batch > 0 && !kv_indices)) return MI_ERR_INVALID;
   if (token_map_len > 0 && (!token_to_page || !token_to_cache)) return MI_ERR_INVALID;
@@ -765,7 +805,10 @@ static int prefill_plan_impl(const int32_t* qo_indptr, const int32_t* kv_indptr,
   const int grid = 2 + (token_map_len + 1023) / 1024;
   if (host)
     hipLaunchKernelGGL(prefill_plan_host_kernel, dim3(grid), dim3(1024), 0, (hipStream_t)stream, a, d, m, *host);
-  else
+  else if (pinned) {
+    pinned->copy_blocks = (pinned->num_indices + 1023) / 1024;
+    hipLaunchKernelGGL(prefill_plan_pinned_kernel, dim3(grid + pinned->copy_blocks), dim3(1024), 0, (hipStream_t)stream, a, d, m, *pinned);
+  } else
     hipLaunchKernelGGL(prefill_plan_kernel, dim3(grid), dim3(1024), 0, (hipStream_t)stream, a, d, m);
   MI_CHECK_LAUNCH();
   return MI_OK;
@@ -781,7 +824,7 @@ extern "C" int mi_prefill_plan(const int32_t* qo_indptr, const int32_t* kv_indpt
                                int64_t workspace_bytes, void* stream) {
   return mi::prefill_plan_impl(qo_indptr, kv_indptr, kv_indices, last_page_len, batch, max_qo_tokens, page_size,
                                num_qo_heads, num_kv_heads, head_dim, token_to_page, token_to_cache, token_map_len,
-                               workspace, workspace_bytes, nullptr, stream);
+                               workspace, workspace_bytes, nullptr, nullptr, stream);
 }
 
 extern "C" int mi_prefill_plan_host(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host,
@@ -800,9 +843,22 @@ extern "C" int mi_prefill_plan_host(const int32_t* qo_indptr_host, const int32_t
   if (st != MI_OK) return st;
   return mi::prefill_plan_impl(qo_indptr, kv_indptr, kv_indices, last_page_len, batch, max_qo_tokens, page_size,
                                num_qo_heads, num_kv_heads, head_dim, token_to_page, token_to_cache, token_map_len,
-                               workspace, workspace_bytes, &m, stream);
+                               workspace, workspace_bytes, &m, nullptr, stream);
 }
 
+extern "C" int mi_prefill_plan_pinned(const int32_t* indices_pinned, int32_t num_indices, int32_t* qo_indptr,
+                                      int32_t* kv_indptr, int32_t* kv_indices, int32_t* last_page_len, int32_t batch,
+                                      int32_t max_qo_tokens, int32_t page_size, int32_t num_qo_heads,
+                                      int32_t num_kv_heads, int32_t head_dim, int64_t* token_to_page,
+                                      int64_t* token_to_cache, int32_t token_map_len, void* workspace,
+                                      int64_t workspace_bytes, void* stream) {
+  if (batch > MI_PLAN_PINNED_BATCH) return MI_ERR_UNSUPPORTED;
+  if (num_indices < 0 || !indices_pinned || !mi::device_reachable(indices_pinned)) return MI_ERR_INVALID;
+  mi::PfPinned m{indices_pinned, num_indices, 0, qo_indptr, kv_indptr, last_page_len, kv_indices};
+  return mi::prefill_plan_impl(qo_indptr, kv_indptr, kv_indices, last_page_len, batch, max_qo_tokens, page_size,
+                               num_qo_heads, num_kv_heads, head_dim, token_to_page, token_to_cache, token_map_len,
+                               workspace, workspace_bytes, nullptr, &m, stream);
+}
 
 namespace mi {
 

@@ -152,7 +152,7 @@ def _host_args(parts: list[torch.Tensor]) -> list[torch.Tensor] | None:
 
 
 def _pinned_args(parts: list[torch.Tensor], n_req: int) -> bool:
-    """Whether a plan launch can read these CPU tensors from pinned memory (``mi_decode_plan_pinned``)."""
+    """Whether a plan launch can read these CPU tensors from pinned memory (``mi_*_plan_pinned``)."""
     return (sum(t.shape[0] for t in parts) <= _lib.PinnedRing.VALUES and 0 < n_req <= _lib.PLAN_PINNED_BATCH
             and all(t.dim() == 1 and t.shape[0] for t in parts) and not torch.cuda.is_current_stream_capturing())
 
@@ -528,8 +528,9 @@ class PagedPrefillWrapper(_FusedRopeAppend):
         else:
             dests = [None] * 4
         host = _host_args(srcs) if on_cpu else None
-        if host is not None:
-            qo, indptr, indices, last = dests if self.use_cuda_graph else _carve(host, dev)
+        pinned = on_cpu and host is None and _pinned_args(srcs, n_req)
+        if host is not None or pinned:
+            qo, indptr, indices, last = dests if self.use_cuda_graph else _carve(srcs, dev)
         elif on_cpu:
             qo, indptr, indices, last = self._staging.upload([t.to(torch.int32) for t in srcs], dev, dests)
         else:
@@ -553,6 +554,11 @@ class PagedPrefillWrapper(_FusedRopeAppend):
         if host is not None:
             _lib.check(_lib.lib().mi_prefill_plan_host(*[t.data_ptr() for t in host], host[2].shape[0], *args),
                        "mi_prefill_plan_host")
+        elif pinned:
+            n_idx = paged_kv_indices.shape[0]
+            _lib.pinned_ring(dev).launch(
+                (qo_indptr, paged_kv_indptr, paged_kv_last_page_len, paged_kv_indices), args[-1],
+                lambda at: _lib.check(_lib.lib().mi_prefill_plan_pinned(at, n_idx, *args), "mi_prefill_plan_pinned"))
         else:
             _lib.check(_lib.lib().mi_prefill_plan(*args), "mi_prefill_plan")
         self._retired = self._indptr  # a run() of the previous plan may still read its arrays on another stream

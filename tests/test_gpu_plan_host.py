@@ -1,4 +1,4 @@
-"""GPU: plans whose CPU index tensors travel in the launch argument.
+"""GPU: plans whose CPU index tensors travel in the launch argument or pinned memory.
 
 At the argument's limit of 800 values and one beyond it (the staged copy),
 plan() must leave the same arrays on the device, the same token map and write
@@ -110,3 +110,32 @@ def test_decode_plan_pinned(gpu, batch, values, graph):
     for a, b in zip(*got):
         assert torch.equal(a, b)
     assert got[0][3].cpu().tolist() == indices.tolist()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("batch,values", [(1, 801), (40, 5000), (1024, 16384), (40, 16385), (1025, 16384)])
+def test_prefill_plan_pinned(gpu, batch, values, graph):
+    """The same for ragged plans, whose tiles, split-KV items and token map all come from the pinned rows."""
+    hq, hkv, d, ps = 8, 2, 128, 16
+    log(f"prefill plan pinned batch={batch} values={values} graph={graph}")
+    lens = _lens(batch, values, 3 * batch + 2, ps)
+    new = [min(n, 1 + 37 * (i % 3)) for i, n in enumerate(lens)]  # short-query and tiled requests
+    qo, indptr, indices, last = custom_batch(lens, ps, 17000, 3, new_lens=new)
+    assert len(qo) + len(indptr) + len(indices) + len(last) == values
+    cache = torch.randn(17000, 2, ps, hkv, d, device=gpu, dtype=torch.bfloat16)
+    q = torch.randn(sum(new), hq, d, device=gpu).to(torch.bfloat16)
+    got = []
+    for dev, dtype in (("cpu", torch.int64), (gpu, torch.int32)):
+        fixed = ({"batch_size": batch, "max_num_pages": 17000, "max_total_tokens": sum(new) + 5, "use_cuda_graph": True}
+                 if graph else {})
+        w = FlashInferPrefillWrapper(workspace(gpu), hq, hkv, d, ps, device=gpu, **fixed)
+        other = [torch.as_tensor(x).to(dev, dtype) for x in (qo, indptr, indices[::-1].copy(), last)]
+        parts = [torch.as_tensor(x).to(dev, dtype) for x in (qo, indptr, indices, last)]
+        for _ in range(2 * _lib.PinnedRing.SLOTS):
+            w.plan(*other)
+            w.plan(*parts)
+        out = w.run(q, cache)
+        got.append((out, w.token_to_page, w.token_to_cache, w._qo, w._indptr, w._indices[: len(indices)], w._last))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    assert got[0][5].cpu().tolist() == indices.tolist()
