@@ -404,7 +404,9 @@ __device__ inline void prefill_plan_body(const PfPlanArgs& a) {
     for (int j0 = 0; j0 < total; j0 += 1024) {
       const int j = j0 + tid;
       int cost = 0, r = 0, row0 = 0;
-      if (j < total) {
+      // only listed tiles are priced: the prefix ends with the cost of the last of them
+      const bool listed = j < total && carry + j < max_tiles;
+      if (listed) {
         int lo = 0, hi = nreq - 1;  // last request whose first tile is <= j (it has tiles)
         while (lo < hi) {
           const int mid = (lo + hi + 1) >> 1;
@@ -417,7 +419,7 @@ __device__ inline void prefill_plan_body(const PfPlanArgs& a) {
       }
       int tot_cost;
       const int cum = block_exclusive_scan_1024(cost, tot_cost, smem);
-      if (j < total && carry + j < max_tiles) {
+      if (listed) {
         mine = make_int2(base + r, row0);
         a.tiles[carry + j] = mine;
         a.tcum[carry + j] = carry_cost + cum;
@@ -431,7 +433,7 @@ __device__ inline void prefill_plan_body(const PfPlanArgs& a) {
   }
   const int listed = min(carry, max_tiles);
   if (tid == 0) {
-    a.tcum[listed] = carry_cost;  // truncated lists keep a consistent prefix end
+    a.tcum[listed] = carry_cost;
     if (listed <= 1024) s_cum[listed] = carry_cost;
   }
   __threadfence_block();
