@@ -792,7 +792,8 @@ int mi_decode_plan_pinned(const int32_t* indices_pinned, int32_t num_indices, in
                                     num_kv_heads, head_dim, kv_locations, workspace, workspace_bytes, 0, &pp);
   if (st != MI_OK) return st;
   if (batch > MI_PLAN_PINNED_BATCH) return MI_ERR_UNSUPPORTED;
-  if (num_indices < 0 || !indices_pinned || !device_reachable(indices_pinned)) return MI_ERR_INVALID;
+  if (num_indices < 0 || (num_indices > 0 && !kv_indices)) return MI_ERR_INVALID;  // copied also without requests
+  if (!indices_pinned || !device_reachable(indices_pinned)) return MI_ERR_INVALID;
   const PinnedIndices m{indices_pinned, num_indices, kv_indptr, kv_indices, last_page_len};
   const int copies = num_indices < 64 * 1024 ? (num_indices + 1023) / 1024 : 64;
   hipLaunchKernelGGL(decode_plan_pinned_kernel, dim3(1 + copies), dim3(1024), 0, (hipStream_t)stream, pp, m);

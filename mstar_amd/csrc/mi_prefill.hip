@@ -856,7 +856,8 @@ extern "C" int mi_prefill_plan_pinned(const int32_t* indices_pinned, int32_t num
                                       int64_t* token_to_cache, int32_t token_map_len, void* workspace,
                                       int64_t workspace_bytes, void* stream) {
   if (batch > MI_PLAN_PINNED_BATCH) return MI_ERR_UNSUPPORTED;
-  if (num_indices < 0 || !indices_pinned || !mi::device_reachable(indices_pinned)) return MI_ERR_INVALID;
+  if (num_indices < 0 || (num_indices > 0 && !kv_indices)) return MI_ERR_INVALID;  // copied also without requests
+  if (!indices_pinned || !mi::device_reachable(indices_pinned)) return MI_ERR_INVALID;
   mi::PfPinned m{indices_pinned, num_indices, 0, qo_indptr, kv_indptr, last_page_len, kv_indices};
   return mi::prefill_plan_impl(qo_indptr, kv_indptr, kv_indices, last_page_len, batch, max_qo_tokens, page_size,
                                num_qo_heads, num_kv_heads, head_dim, token_to_page, token_to_cache, token_map_len,
