@@ -301,7 +301,8 @@ int mi_prefill_plan(const int32_t* qo_indptr, const int32_t* kv_indptr,
  * four (three) arrays travel in the launch argument, and the launch writes them
  * to the device arrays that the run call will read before it plans, so that a
  * step with few pages needs no copy of its own.  num_indices: elements of
- * kv_indices.  At most MI_PLAN_HOST_ARGS int32 values in all
+ * kv_indices, within which kv_indptr has to end (MI_ERR_INVALID otherwise).
+ * At most MI_PLAN_HOST_ARGS int32 values in all
  * (MI_ERR_UNSUPPORTED beyond: copy them and call the other entry point); the
  * host arrays are not read after the call returns.  No counterpart in the
  * reference, which copies its index tensors one by one. */
@@ -320,7 +321,7 @@ int mi_decode_plan_host(const int32_t* kv_indptr_host, const int32_t* kv_indices
                         void* workspace, int64_t workspace_bytes, void* stream);
 /* mi_decode_plan for more values than an argument holds: [kv_indptr (batch + 1) |
  * last_page_len (batch) | kv_indices (num_indices)] in pinned host memory
- * (allocated through HIP; MI_ERR_INVALID otherwise), read by the launch itself
+ * (kv_indptr must end within num_indices, which is not checked; allocated through HIP; MI_ERR_INVALID otherwise), read by the launch itself
  * and to be left alone until it has run.  batch at most MI_PLAN_PINNED_BATCH
  * (MI_ERR_UNSUPPORTED beyond). */
 #define MI_PLAN_PINNED_BATCH 1024

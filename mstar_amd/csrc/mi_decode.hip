@@ -596,6 +596,7 @@ static int decode_plan_host_impl(const int32_t* const* src, int32_t num_indices,
   HostIndices m;
   st = host_indices(src, len, dst, 3, &m);
   if (st != MI_OK) return st;
+  if (src[0][batch] > num_indices) return MI_ERR_INVALID;  // pages past the argument's
   hipLaunchKernelGGL(decode_plan_host_kernel, dim3(1), dim3(1024), 0, stream, pp, m);
   MI_CHECK_LAUNCH();
   return MI_OK;

@@ -844,6 +844,7 @@ extern "C" int mi_prefill_plan_host(const int32_t* qo_indptr_host, const int32_t
   mi::HostIndices m;
   const int st = mi::host_indices(src, len, dst, 4, &m);
   if (st != MI_OK) return st;
+  if (kv_indptr_host[batch] > num_indices) return MI_ERR_INVALID;  // pages past the argument's
   return mi::prefill_plan_impl(qo_indptr, kv_indptr, kv_indices, last_page_len, batch, max_qo_tokens, page_size,
                                num_qo_heads, num_kv_heads, head_dim, token_to_page, token_to_cache, token_map_len,
                                workspace, workspace_bytes, &m, nullptr, stream);

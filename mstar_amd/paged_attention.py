@@ -140,21 +140,26 @@ class _Staging:
         return outs
 
 
+def _launch_reads(parts: list[torch.Tensor], indptr: torch.Tensor, indices: torch.Tensor) -> bool:
+    """Whether a plan launch may read these CPU tensors by itself.  Not an empty
+    part, nor page lists that end past ``indices`` (in graph mode the rest is what
+    the static buffer holds), nor a plan under graph capture: those keep the
+    staged copy, which is recorded there."""
+    return (all(t.dim() == 1 and t.shape[0] for t in parts) and int(indptr.numpy()[-1]) <= indices.shape[0]
+            and not torch.cuda.is_current_stream_capturing())
+
+
 def _host_args(parts: list[torch.Tensor]) -> list[torch.Tensor] | None:
     """The contiguous int32 CPU tensors of a plan whose indices travel in the
-    launch argument (``mi_*_plan_host``), or None: too many values, an empty
-    part, or a plan under graph capture (its staged copy is recorded there)."""
-    if sum(t.shape[0] for t in parts) > _lib.PLAN_HOST_ARGS or not all(t.dim() == 1 and t.shape[0] for t in parts):
-        return None
-    if torch.cuda.is_current_stream_capturing():
+    launch argument (``mi_*_plan_host``), or None: too many values."""
+    if sum(t.shape[0] for t in parts) > _lib.PLAN_HOST_ARGS:
         return None
     return [t if t.dtype == torch.int32 and t.is_contiguous() else t.to(torch.int32).contiguous() for t in parts]
 
 
 def _pinned_args(parts: list[torch.Tensor], n_req: int) -> bool:
     """Whether a plan launch can read these CPU tensors from pinned memory (``mi_*_plan_pinned``)."""
-    return (sum(t.shape[0] for t in parts) <= _lib.PinnedRing.VALUES and 0 < n_req <= _lib.PLAN_PINNED_BATCH
-            and all(t.dim() == 1 and t.shape[0] for t in parts) and not torch.cuda.is_current_stream_capturing())
+    return sum(t.shape[0] for t in parts) <= _lib.PinnedRing.VALUES and 0 < n_req <= _lib.PLAN_PINNED_BATCH
 
 
 def _carve(parts: list[torch.Tensor], device: torch.device) -> list[torch.Tensor]:
@@ -311,8 +316,9 @@ class PagedDecodeWrapper(_FusedRopeAppend):
         nv = self.enable_nvtx
         with trace_range(nv, "flashinfer.decode.metadata_h2d"):
             on_cpu = all(t.is_cpu for t in srcs)
-            host = _host_args(srcs) if on_cpu else None
-            pinned = on_cpu and host is None and _pinned_args(srcs, n_req)
+            direct = on_cpu and _launch_reads(srcs, paged_kv_indptr, paged_kv_indices)
+            host = _host_args(srcs) if direct else None
+            pinned = direct and host is None and _pinned_args(srcs, n_req)
             if host is not None or pinned:
                 indptr, indices, last = dests if self.use_cuda_graph else _carve(srcs, dev)
             elif on_cpu:
@@ -527,8 +533,9 @@ class PagedPrefillWrapper(_FusedRopeAppend):
                      self._paged_kv_last_page_len_buf]
         else:
             dests = [None] * 4
-        host = _host_args(srcs) if on_cpu else None
-        pinned = on_cpu and host is None and _pinned_args(srcs, n_req)
+        direct = on_cpu and _launch_reads(srcs, paged_kv_indptr, paged_kv_indices)
+        host = _host_args(srcs) if direct else None
+        pinned = direct and host is None and _pinned_args(srcs, n_req)
         if host is not None or pinned:
             qo, indptr, indices, last = dests if self.use_cuda_graph else _carve(srcs, dev)
         elif on_cpu:

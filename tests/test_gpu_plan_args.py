@@ -5,8 +5,9 @@ import ctypes
 import pytest
 import torch
 
-from gpu_helpers import log, workspace
+from gpu_helpers import custom_batch, log, workspace
 from mstar_amd import _lib
+from mstar_amd.paged_attention import FlashInferDecodeWrapper, FlashInferPrefillWrapper
 
 pytestmark = pytest.mark.gpu
 
@@ -34,3 +35,39 @@ def test_pinned_plans_without_requests(gpu, num_indices, kv_indices, status):
     torch.cuda.synchronize()
     if status == 0 and num_indices:
         assert dst[3, :5].tolist() == src[2:7].tolist()
+
+
+@pytest.mark.parametrize("kind", ["decode", "prefill"])
+@pytest.mark.parametrize("pages", [40, 2000])  # in the launch argument; in pinned memory
+def test_page_lists_longer_than_the_indices(gpu, kind, pages):
+    """A graph-mode plan whose kv_indptr ends past the given indices takes the rest
+    from the static buffer, whichever way the arrays come in."""
+    log(f"{kind} plan: page lists end 5 past {pages} indices")
+    qo, indptr, indices, last = custom_batch([16 * (pages // 2), 16 * (pages - pages // 2) + 75], 16, pages + 10, 3,
+                                             new_lens=[1, 1] if kind == "decode" else [20, 90])
+    assert indptr[-1] == pages + 5
+    meta = [torch.as_tensor(x) for x in (qo, indptr, indices[:pages], last)]
+    got = []
+    for dev in ("cpu", gpu):
+        fixed = {"batch_size": 2, "max_num_pages": pages + 10, "use_cuda_graph": True, "device": gpu}
+        if kind == "decode":
+            w = FlashInferDecodeWrapper(workspace(gpu), 8, 2, 128, 16, **fixed)
+        else:
+            w = FlashInferPrefillWrapper(workspace(gpu), 8, 2, 128, 16, max_total_tokens=110, **fixed)
+        w._paged_kv_indices_buf.copy_(torch.arange(pages + 10))
+        w.plan(*(t.to(dev) for t in meta[kind == "decode":]))
+        got.append([w._indices, w.kv_cache_locations] if kind == "decode" else
+                   [w._indices, w.token_to_page, w.token_to_cache])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
+def test_host_plans_refuse_page_lists_past_the_argument(gpu):
+    log("host plans: kv_indptr ends past num_indices")
+    L, ws = _lib.lib(), workspace(gpu, 64 << 20)
+    i32 = ctypes.c_int32 * 2
+    indptr, qo, idx, last = i32(0, 3), i32(0, 1), i32(4, 5), i32(1, 0)
+    dst = [ctypes.c_void_p(t.data_ptr()) for t in torch.zeros(4, 16, dtype=torch.int32, device=gpu)]
+    tail = (ctypes.c_void_p(ws.data_ptr()), ws.numel(), _lib.stream_ptr(gpu))
+    assert L.mi_decode_plan_host(indptr, idx, last, 2, *dst[1:], 1, 16, 8, 2, 128, None, *tail) == INVALID
+    assert L.mi_prefill_plan_host(qo, indptr, idx, last, 2, *dst, 1, 1, 16, 8, 2, 128, None, None, 0, *tail) == INVALID
