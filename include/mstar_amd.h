@@ -276,10 +276,13 @@ int mi_kv_append(const mi_paged_kv* kv, const void* k, const void* v, int32_t sr
  * tiles of the long-query requests, and the merge of those that the plan has
  * cut into key pieces), the merges of both in one launch where the types
  * allow.  The halves take the same arguments and write disjoint output rows;
- * after the plan they may run in either order or on two streams.  They have no separate counterpart in the reference.
+ * after the plan they may run in either order or on two streams.  They have no
+ * separate counterpart in the reference.
  * ------------------------------------------------------------------------ */
 /* The size with room for the partials of cut tiles; a smaller workspace that
- * still holds the plan leaves the tiles uncut. */
+ * still holds the plan leaves the tiles uncut.  Runs take the same workspace;
+ * one that states fewer bytes than its plan did, but enough for the plan, has
+ * the tiles computed whole. */
 int64_t mi_prefill_workspace_bytes(int32_t batch, int32_t max_qo_tokens, int32_t num_qo_heads,
                                    int32_t num_kv_heads, int32_t head_dim);
 /* Which requests of a plan of this shape are short-query requests (run by

@@ -46,8 +46,8 @@ constexpr int kShortRows = kShortRowsMax;  // qo_len * group <= 16 -> decode ker
 // is left) piece list | split tile list | piece partials (lse, o).
 // Header words: [kPfTiles] tiles, [kPfUnits] units (tiles x kv-heads, or
 // pieces x kv-heads when tiles are split), [kPfPieces] pieces per kv-head (0:
-// no tile is split), [kPfSplitTiles] split tiles, [kPfCuts + x] first unit of
-// XCD x's queue (x = 0..8, [16] = units).
+// no tile is split), [kPfSplitTiles] split tiles, [kPfSlots] partials,
+// [kPfCuts + x] first unit of XCD x's queue (x = 0..8, [16] = units).
 struct PrefillLayout {
   int64_t hdr, ctr, tiles, tcum, order, split;
   int32_t max_tiles;
@@ -56,6 +56,8 @@ struct PrefillLayout {
 // What a split of tiles into key pieces needs, behind the decode split plan:
 // as many partials as fit the workspace, up to kPfMaxParts (three rounds of
 // one piece per CU; a split of more pieces never paid).  parts == 0: no room.
+// Every table has its place whatever the workspace's size, so a run finds them
+// also where it is given another size than the plan was.
 constexpr int32_t kPfMaxParts = 768;
 struct PfSplitLayout {
   int64_t pieces, split_tiles, lse, o, total;
@@ -63,21 +65,17 @@ struct PfSplitLayout {
 };
 
 static PfSplitLayout pf_split_layout(int64_t base, int32_t max_tiles, int32_t nkv, int32_t head_dim, int64_t ws_avail) {
-  PfSplitLayout P{};
-  P.total = base;
-  const int64_t rows = pf_rows(head_dim);
-  const int64_t per_part = 16 + 16 + 4 * rows + 4 * rows * head_dim;
-  const int64_t fixed = 16LL * max_tiles + 5 * 256;
-  int64_t parts = kPfMaxParts;
-  if (ws_avail >= 0 && (ws_avail - base - fixed) / per_part < parts) parts = (ws_avail - base - fixed) / per_part;
-  if (parts < 2 * nkv) return P;
-  P.parts = (int32_t)parts;
-  P.max_pieces = max_tiles + P.parts;
+  PfSplitLayout P;
+  const int64_t rows = pf_rows(head_dim), per_part = 4 * rows * head_dim;
+  P.max_pieces = max_tiles + kPfMaxParts;
   P.pieces = mi_align_up(base, 256);
   P.split_tiles = mi_align_up(P.pieces + 16LL * P.max_pieces, 256);
-  P.lse = mi_align_up(P.split_tiles + 16LL * P.parts, 256);
-  P.o = mi_align_up(P.lse + 4 * rows * P.parts, 256);
-  P.total = mi_align_up(P.o + 4 * rows * head_dim * P.parts, 256);
+  P.lse = mi_align_up(P.split_tiles + 16LL * kPfMaxParts, 256);
+  P.o = mi_align_up(P.lse + 4 * rows * kPfMaxParts, 256);
+  int64_t parts = kPfMaxParts;
+  if (ws_avail >= 0 && ws_avail < P.o + parts * per_part) parts = ws_avail > P.o ? (ws_avail - P.o) / per_part : 0;
+  P.parts = parts < 2 * nkv ? 0 : (int32_t)parts;
+  P.total = P.parts ? P.o + P.parts * per_part : base;
   return P;
 }
 
@@ -98,7 +96,7 @@ static PrefillLayout prefill_layout(int32_t batch, int32_t max_qo_tokens, int32_
   return L;
 }
 
-// The split layout of a plan or run call (shapes only, so the two agree).
+// The split layout of a plan or run call: from its shapes, and how much of it there is room for.
 static PfSplitLayout pf_split_of(const PrefillLayout& L, int32_t batch, int32_t group, int32_t nkv, int32_t head_dim,
                                  int64_t ws_bytes) {
   const bool pair = pair_heads(nullptr, batch, nkv, group, head_dim, true);
@@ -367,6 +365,7 @@ __device__ inline void pf_deal(const PfPlanArgs& a, int n_tiles, int cap, int mc
     a.hdr[kPfUnits] = np * a.nkv;
     a.hdr[kPfPieces] = np;
     a.hdr[kPfSplitTiles] = carry_split;
+    a.hdr[kPfSlots] = a.nkv * carry_slots;
   }
 }
 
@@ -446,6 +445,7 @@ __device__ inline void prefill_plan_body(const PfPlanArgs& a) {
     a.hdr[kPfTiles] = n_tiles;
     a.hdr[kPfPieces] = 0;
     a.hdr[kPfSplitTiles] = 0;
+    a.hdr[kPfSlots] = 0;
   }
   const int32_t* tcum = a.tcum;
   auto prefix = [&](int t) { return n_tiles <= 1024 ? s_cum[t] : tcum[t]; };
@@ -620,7 +620,7 @@ MI_DEVICE void prefill_merge_body(const PrefillParams& p, int first_wave, int wa
   constexpr float kNegInf = -__builtin_inff();
   const int nkv = p.num_kv_heads, G = p.group;
   const int lane = lane_id(), col = lane & 15, grp = lane >> 4;
-  const int total = p.hdr[kPfSplitTiles] * nkv * NG * 4;
+  const int total = pf_fits(p) ? p.hdr[kPfSplitTiles] * nkv * NG * 4 : 0;
   for (int w = uniform(first_wave + ((int)threadIdx.x >> 6)); w < total; w += waves) {
     const int part = w & 3, rgi = (w >> 2) % NG, th = (w >> 2) / NG;
     const int h = th % nkv;
@@ -968,6 +968,7 @@ static int prefill_run_impl(const void* q, int32_t q_dtype, int64_t q_stride_tok
   pp.split_tiles = (const int4*)(ws + P.split_tiles);
   pp.part_lse = (float*)((uint8_t*)workspace + P.lse);
   pp.part_o = (float4*)((uint8_t*)workspace + P.o);
+  pp.parts = P.parts;
   pp.out = out;
   pp.out_stride_tok = out_stride_token;
   pp.out_stride_head = out_stride_head;

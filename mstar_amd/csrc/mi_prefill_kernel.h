@@ -23,7 +23,7 @@ constexpr int kPfKeys = 32;                // keys per K/V tile
 constexpr int kPfTileCap = 1024;           // tiles whose row-group addresses are staged in LDS at a time
 constexpr int kCtrStride = 32;  // one 128-byte line per XCD counter
 // Header words of the prefill plan (see mi_prefill.hip).
-enum { kPfTiles = 0, kPfUnits, kPfPieces, kPfSplitTiles, kPfCuts = 8 };
+enum { kPfTiles = 0, kPfUnits, kPfPieces, kPfSplitTiles, kPfSlots, kPfCuts = 8 };
 constexpr int kPfMaxPieces = 1024;  // key pieces of one tile (their index and count share an int)
 
 // ------------------------------------------------------------ attention
@@ -48,6 +48,7 @@ struct PrefillParams {
   const int4* split_tiles;   // (request, first row, pieces, first slot)
   float4* part_o;            // [slot][row group of 16][D/16][64 lanes], normalised
   float* part_lse;           // [slot][tile rows]
+  int32_t parts;             // slots that the run's workspace has room for
   void* out;
   int64_t out_stride_tok, out_stride_head;
   int32_t num_kv_heads, group, page_size, causal;
@@ -57,8 +58,13 @@ struct PrefillParams {
 // A unit's tile and, for a piece of a split tile, which part of the tile's
 // key steps it covers and where its partial goes.
 struct PfUnit {
-  int h, b, row0, k, n, slot;  // slot: the piece's own partial (n > 1)
+  int h, b, row0, k, n, slot;  // slot: the piece's own partial (n > 1); n == 0: nothing to do
 };
+
+// Whether the run's workspace holds the partials of the plan's cut.  One that
+// is smaller than the plan's computes the tiles whole instead, each as its
+// first piece's unit.
+MI_DEVICE bool pf_fits(const PrefillParams& p) { return p.hdr[kPfSlots] <= p.parts; }
 
 // Dealt plans: np pieces per kv-head, heaviest first, dealt to the 8 queues so
 // that each XCD sees as few heads as an even deal allows: 8 / nkv XCDs per
@@ -116,6 +122,7 @@ MI_DEVICE int pf_claim(const PrefillParams& p) {
 MI_DEVICE PfUnit pf_unit(const PrefillParams& p, int claim) {
   PfUnit r;
   const int x = claim & 7, i = claim >> 3;
+  const bool fits = pf_fits(p);  // read with the next word
   if (p.hdr[kPfPieces] == 0) {
     const int nt = p.hdr[kPfTiles];
     const int unit = p.order[p.hdr[kPfCuts + x] + i];
@@ -135,6 +142,7 @@ MI_DEVICE PfUnit pf_unit(const PrefillParams& p, int claim) {
     r.k = pe.z & 0xffff;
     r.n = pe.z >> 16;
     r.slot = pe.w + r.h * r.n + r.k;
+    if (!fits) r.n = r.k == 0 ? 1 : 0;
   }
   return r;
 }
@@ -245,6 +253,7 @@ __global__ __launch_bounds__(64 * pf_waves(D)) void prefill_kernel(PrefillParams
   const int n_kt = kv_end > 0 ? (kv_end + KEYS - 1) / KEYS : 0;
   // key steps of this unit: all of the tile's, or its piece's share
   const int kt0 = un.n > 1 ? un.k * n_kt / un.n : 0, kt1 = un.n > 1 ? (un.k + 1) * n_kt / un.n : n_kt;
+  if (un.n == 0) continue;  // uniform; no wait for the unit's entry ahead of the loads above
 
   float kscale = 1.f, vscale = 1.f;
   if constexpr (FP8) {

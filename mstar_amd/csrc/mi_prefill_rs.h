@@ -121,6 +121,7 @@ __global__ __launch_bounds__(512) void prefill_rs_kernel(PrefillParams p) {
       const int n_kt = kv_end > 0 ? (kv_end + KEYS - 1) / KEYS : 0;
       // key steps of this unit: all of the tile's, or its piece's share
       const int kt0 = un.n > 1 ? un.k * n_kt / un.n : 0, kt1 = un.n > 1 ? (un.k + 1) * n_kt / un.n : n_kt;
+      if (un.n == 0) continue;  // uniform; no wait for the unit's entry ahead of the loads above
 
       float kscale = 1.f, vscale = 1.f;
       if constexpr (FP8) {

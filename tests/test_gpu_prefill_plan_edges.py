@@ -3,7 +3,7 @@
 import pytest
 import torch
 
-from gpu_helpers import custom_batch, log
+from gpu_helpers import custom_batch, log, random_cache
 from mstar_amd import _lib
 from mstar_amd.paged_attention import FlashInferPrefillWrapper
 
@@ -20,11 +20,11 @@ def _hdr(ws):
 def test_tiles_past_the_stated_tokens_are_not_priced(gpu, stated):
     """Device index tensors with more query tokens than the caller states: the
     tiles beyond the list are left out of the costs as well, so the cut of the
-    listed ones keeps to the workspace's room for partials (about 16 here; priced
+    listed ones keeps to the workspace's room for partials (24 here; priced
     with the last listed tile carrying the others' 1600-1700 key steps, it had 90
     to 106)."""
     log(f"prefill plan: 320 query tokens, {stated} stated")
-    hq, hkv, d, ps, room = 16, 1, 128, 16, 16
+    hq, hkv, d, ps, room = 16, 1, 128, 16, 24
     meta = [torch.as_tensor(x).to(gpu) for x in custom_batch([3200], ps, 210, 3, new_lens=[320])]
     size = _lib.lib().mi_prefill_workspace_bytes(1, stated, hq, hkv, d) - (768 - room) * PART_O
     guard = torch.full((size + (4 << 20),), 0x5A, dtype=torch.uint8, device=gpu)
@@ -33,5 +33,50 @@ def test_tiles_past_the_stated_tokens_are_not_priced(gpu, stated):
     tiles, _, pieces, split = _hdr(guard)[:4]
     log(f"  tiles={tiles} pieces={pieces} split tiles={split}")
     assert tiles == -(-stated * hq // 256) + 1
-    assert tiles <= pieces <= tiles + 2 * room and split <= tiles
+    assert tiles <= pieces <= tiles + room and split <= tiles
     assert bool((guard[size:] == 0x5A).all())
+
+
+@pytest.mark.parametrize("heads,fp8", [((8, 2, 128), False), ((8, 2, 128), True), ((16, 4, 64), False),
+                                       ((8, 1, 256), False), ((8, 1, 256), True)])
+def test_runs_that_state_another_workspace_size(gpu, heads, fp8):
+    """A plan and its runs given different sizes of one workspace, each of which
+    holds the plan: tiles are computed whole wherever the run's size has no room
+    for the plan's partials, and the bits are those of equal sizes."""
+    hq, hkv, d = heads
+    log(f"workspace sizes of plan and run {heads} fp8={fp8}")
+    ps, kv, new = 16, [3000, 700, 900], [90, 50, 1]  # cut tiles, and a short-query request
+    meta = custom_batch(kv, ps, 300, 3, new_lens=new)
+    cache = random_cache(300, ps, hkv, d, 5).to(gpu)
+    scales = (None, None)
+    if fp8:
+        cache, scales = cache.to(torch.float8_e4m3fn), (torch.full((hkv,), 0.5, device=gpu),) * 2
+    q = torch.randn(sum(new), hq, d, generator=torch.Generator().manual_seed(6)).to(torch.bfloat16).to(gpu)
+    full = _lib.lib().mi_prefill_workspace_bytes(len(kv), sum(new), hq, hkv, d)
+    part = 4 * d * (128 if d == 256 else 256)
+    roomy, few, none = full, full - (768 - 2 * hkv) * part, full - 768 * part
+    ws = torch.empty(full, dtype=torch.uint8, device=gpu)
+
+    def go(planned, ran, serial):
+        w = FlashInferPrefillWrapper(ws[:planned], hq, hkv, d, ps, device=gpu)
+        w.plan(*(torch.as_tensor(x) for x in meta))
+        cut = _hdr(ws)[3] > 0
+        w._workspace, w._serial = ws[:ran], serial
+        out = torch.full_like(q, float("nan"))
+        w.run(q, cache, *scales, out=out)
+        again = w.run(q, cache, *scales)
+        assert torch.equal(out, again), "a plan's second run differs"
+        return out, cut
+
+    whole, cut = go(none, none, True)
+    assert not cut
+    cut_out, cut = go(roomy, roomy, True)
+    assert cut and bool(cut_out.isfinite().all())
+    for serial in (True, False):
+        assert torch.equal(go(roomy, roomy, serial)[0], cut_out)
+        for planned, ran in ((roomy, few), (roomy, none), (none, roomy), (none, few)):
+            out, cut = go(planned, ran, serial)
+            assert cut == (planned == roomy)
+            assert torch.equal(out, whole), (planned, ran, serial)
+        small, _ = go(few, few, serial)
+        assert torch.equal(go(few, roomy, serial)[0], small)
