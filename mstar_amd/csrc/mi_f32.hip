@@ -371,6 +371,9 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(DecodeParams p, F32
   const int last_qtok = (row_wg + rows_wg - 1) / G;
   const int kv_end = p.causal ? min(kv_len, kv_len - qo_len + last_qtok + 1) : kv_len;
   const int steps = kv_end > 0 ? (kv_end + KT - 1) / KT : 0;
+  // keys that the rows of a wavefront see, and the fewest that those of one do
+  auto end_of = [&](int last_row) { return p.causal ? min(kv_len, kv_len - qo_len + last_row / G + 1) : kv_len; };
+  const int min_end = end_of(row_wg + min(rows_wg, 16) - 1), wave_end = end_of(row_wg + min(rows_wg, 16 * wave + 16) - 1);
 
   const int row = row_wg + 16 * wave + col, qtok = row / G, g = row - qtok * G;
   const bool row_valid = row < qo_len * G;
@@ -427,10 +430,22 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(DecodeParams p, F32
   for (int m = 0; m < VW; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m_run = kNegInf, l_run = 0.f;
 
-  auto compute = [&](int t, int st) {
+  // One key step.  TAIL: it may end past the wavefront's keys, whose 16-key
+  // groups are left out one by one: a masked key's V is multiplied by zero,
+  // which a NaN or Inf in it survives, so a row meets no key beyond its 16-row
+  // block's last group.
+  auto compute = [&](int t, int st, auto tail) {
+    constexpr bool TAIL = decltype(tail)::value;
+    auto used = [&](int k) { return !TAIL || t * KT + 16 * k < wave_end; };  // uniform
+    if (!used(0)) return;
     float sv[NS][4];
 #pragma unroll
     for (int k = 0; k < NS; ++k) {
+      if (!used(k)) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sv[k][r] = kNegInf;
+        continue;
+      }
       f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
       const float4* krun = (const float4*)(lds_k[st] + (16 * k + col) * KRS + KQ * grp * 4);
 #pragma unroll
@@ -473,7 +488,8 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(DecodeParams p, F32
       l_run += (sv[k][0] + sv[k][1]) + (sv[k][2] + sv[k][3]);
     }
 #pragma unroll
-    for (int k = 0; k < NS; ++k)
+    for (int k = 0; k < NS; ++k) {
+      if (!used(k)) continue;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const uint8_t* vrow = lds_v[st] + (16 * k + 4 * grp + r) * D * 4 + 16 * col;
@@ -486,6 +502,7 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(DecodeParams p, F32
           acc[4 * i + 3] = mma_f32(a.w, sv[k][r], acc[4 * i + 3]);
         }
       }
+    }
   };
   static_assert(RUN == 4, "a lane's dims: one float4 per 64");
 
@@ -495,15 +512,18 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(DecodeParams p, F32
     find_pages(1);
     store_step(0, 0);
     __syncthreads();
-    for (int t = 0; t < steps; ++t) {
+    auto step = [&](int t, auto tail) {
       if (t + 1 < steps) {
         load_step();  // step t + 1
         find_pages(t + 2);
       }
-      compute(t, t & 1);
+      compute(t, t & 1, tail);
       if (t + 1 < steps) store_step(t + 1, (t + 1) & 1);  // the stage of step t - 1
       __syncthreads();
-    }
+    };
+    int t = 0;
+    for (const int whole = min_end > 0 ? min_end / KT : 0; t < whole; ++t) step(t, std::false_type{});
+    for (; t < steps; ++t) step(t, std::true_type{});
   }
   const float L = rows4_sum(l_run);
   const float inv = L > 0.f ? 1.f / L : (L == 0.f ? 0.f : __builtin_nanf(""));  // NaN L: keep the row NaN
