@@ -335,9 +335,10 @@ __global__ __launch_bounds__(256) void attend_f32_kernel(DecodeParams p, F32Tile
 // K or V fragment feeds four MFMAs.  attend_f32_kernel<D, true> reads each K/V
 // row from L2 once per 16 rows and keys' quarter instead: on 4 prefixes of
 // 800-1000 tokens at 8 q / 1 kv / 256 its 3.3 GB of L2 reads, not the MFMAs,
-// set the time.  Here the matrix cores are busy 70% of the time: 382 -> 268 us on 4 x 900
-// keys, 69 -> 99 TFLOP/s (without the softmax, with fragments read six ahead or
-// with two key groups per workgroup in opposite phase no faster).
+// set the time: 409 us on 4 x 900 keys, 303 here (88 TFLOP/s).  Bound by the
+// fp32 MFMAs and the vector work beside them, which add up: a step's 64 FMAs
+// into O at head_dim 256 take 7 %, so its address arithmetic, bounds and masks
+// are kept out of the steps that lie wholly within the rows' keys (5 %).
 // S^T, the softmax and O^T use the same operand layouts as there (S^T in two
 // chains over the head_dim); V rows past kv_len are stored as zeros.
 template <int D>
@@ -371,9 +372,9 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(DecodeParams p, F32
   const int last_qtok = (row_wg + rows_wg - 1) / G;
   const int kv_end = p.causal ? min(kv_len, kv_len - qo_len + last_qtok + 1) : kv_len;
   const int steps = kv_end > 0 ? (kv_end + KT - 1) / KT : 0;
-  // keys that the rows of a wavefront see, and the fewest that those of one do
-  auto end_of = [&](int last_row) { return p.causal ? min(kv_len, kv_len - qo_len + last_row / G + 1) : kv_len; };
-  const int min_end = end_of(row_wg + min(rows_wg, 16) - 1), wave_end = end_of(row_wg + min(rows_wg, 16 * wave + 16) - 1);
+  // keys that the wavefront's own 16 rows see
+  const int last_w = row_wg + min(rows_wg, 16 * wave + 16) - 1;
+  const int wave_end = p.causal ? min(kv_len, kv_len - qo_len + last_w / G + 1) : kv_len;
 
   const int row = row_wg + 16 * wave + col, qtok = row / G, g = row - qtok * G;
   const bool row_valid = row < qo_len * G;
@@ -405,23 +406,25 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(DecodeParams p, F32
     }
   };
   f32x4 rk[NL], rv[NL];
+  constexpr int RPC = 256 / CPR;  // rows between a thread's chunks
+  const int64_t own = (int64_t)(tid / CPR) * tok_bytes + 16 * (tid % CPR);
   auto load_step = [&]() {
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
-      const int c = tid + 256 * i, r = (c / CPR) & 15, k = i / CPG;
-      const uint8_t* src = kvb + (int64_t)pg[k] * page_bytes + (int64_t)(slot[k] + r) * tok_bytes + 16 * (c % CPR);
-      rk[i] = *(const f32x4*)src;
-      rv[i] = *(const f32x4*)(src + kvhalf);
+      const int k = i / CPG;
+      const uint8_t* src = kvb + (int64_t)pg[k] * page_bytes + (int64_t)(slot[k] + i % CPG * RPC) * tok_bytes;  // scalar
+      rk[i] = *(const f32x4*)(src + own);
+      rv[i] = *(const f32x4*)(src + kvhalf + own);
     }
   };
-  auto store_step = [&](int t, int st) {
-    const bool tail = (t + 1) * KT > kv_len;
+  auto store_step = [&](int t, int st, auto tail) {
+    uint8_t* kdst = lds_k[st] + tid / CPR * KRS + 16 * (tid % CPR);
+    uint8_t* vdst = lds_v[st] + 16 * tid;
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
-      const int c = tid + 256 * i, r = c / CPR;
-      const bool past = tail && t * KT + r >= kv_len;  // slots past the end hold stale data
-      *(f32x4*)(lds_k[st] + r * KRS + 16 * (c % CPR)) = rk[i];
-      *(f32x4*)(lds_v[st] + r * D * 4 + 16 * (c % CPR)) = past ? f32x4{0.f, 0.f, 0.f, 0.f} : rv[i];
+      *(f32x4*)(kdst + i * RPC * KRS) = rk[i];
+      if (decltype(tail)::value && t * KT + tid / CPR + i * RPC >= kv_len) rv[i] = f32x4{0.f, 0.f, 0.f, 0.f};  // slots past the end hold stale data
+      *(f32x4*)(vdst + i * 16 * 256) = rv[i];
     }
   };
 
@@ -459,7 +462,7 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(DecodeParams p, F32
 #pragma unroll
       for (int r = 0; r < 4; ++r) sv[k][r] = (s0[r] + s1[r]) * sl2;
     }
-    if ((t + 1) * KT > mask_from) {
+    if (TAIL && (t + 1) * KT > mask_from) {
 #pragma unroll
       for (int k = 0; k < NS; ++k)
 #pragma unroll
@@ -469,40 +472,51 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(DecodeParams p, F32
     float ml = kNegInf;  // this lane's share of the row
 #pragma unroll
     for (int k = 0; k < NS; ++k) ml = fmaxf(ml, fmaxf(fmaxf(sv[k][0], sv[k][1]), fmaxf(sv[k][2], sv[k][3])));
-    // The running max is raised only when a score exceeds it by more than 8:
-    // probabilities then stay below 2^8, which costs fp32 no precision, and most
-    // steps need neither the row max across lanes nor a rescale of O.
-    if (__builtin_amdgcn_ballot_w64(ml > m_run + 8.f)) {
-      const float m_new = fmaxf(m_run, rows4_max(ml));
-      const float alpha = m_new > m_run ? fast_exp2(m_run - m_new) : 1.f;
-      m_run = m_new;
-      l_run *= alpha;
-#pragma unroll
-      for (int m = 0; m < VW; ++m) acc[m] *= alpha;
-    }
+    const float m_new = fmaxf(m_run, rows4_max(ml));
+    const float alpha = m_new > m_run ? fast_exp2(m_run - m_new) : 1.f;
+    m_run = m_new;
     const float m_use = m_run == kNegInf ? 0.f : m_run;
+    float ls = 0.f;
 #pragma unroll
     for (int k = 0; k < NS; ++k) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) sv[k][r] = fast_exp2(sv[k][r] - m_use);
-      l_run += (sv[k][0] + sv[k][1]) + (sv[k][2] + sv[k][3]);
+      ls += (sv[k][0] + sv[k][1]) + (sv[k][2] + sv[k][3]);
     }
+    l_run = fmaf(l_run, alpha, ls);
+    // The step's P.V is summed by itself, then added: O is rounded at its own size
+    // once a step.  (Summed key by key into O, with a max that was raised only past
+    // 2^8, 2048 keys were 1.3-1.7x as far from 64 bits as attend_f32_kernel's four
+    // shorter sums over exact maxima.)
+    f32x4 o[2][4];
+    auto add = [&](int i) {
 #pragma unroll
-    for (int k = 0; k < NS; ++k) {
-      if (!used(k)) continue;
+      for (int m = 0; m < 4; ++m)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const uint8_t* vrow = lds_v[st] + (16 * k + 4 * grp + r) * D * 4 + 16 * col;
+        for (int e = 0; e < 4; ++e) acc[4 * i + m][e] = fmaf(acc[4 * i + m][e], alpha, o[i & 1][m][e]);
+    };
+    // at head_dim 256 a group of dims late, so that the matrix core's latency is
+    // not waited for (296 us instead of 300 on 4 x 900 keys; slower below)
+    constexpr int LATE = D > 128 ? 1 : 0;
 #pragma unroll
-        for (int i = 0; i < NV; ++i) {  // elements 4i..4i+3 of the lane: dims dim_of(RUN, col, 4i)
-          const float4 a = *(const float4*)(vrow + 256 * i);
-          acc[4 * i] = mma_f32(a.x, sv[k][r], acc[4 * i]);
-          acc[4 * i + 1] = mma_f32(a.y, sv[k][r], acc[4 * i + 1]);
-          acc[4 * i + 2] = mma_f32(a.z, sv[k][r], acc[4 * i + 2]);
-          acc[4 * i + 3] = mma_f32(a.w, sv[k][r], acc[4 * i + 3]);
+    for (int i = 0; i < NV; ++i) {  // elements 4i..4i+3 of the lane: dims dim_of(RUN, col, 4i)
+#pragma unroll
+      for (int m = 0; m < 4; ++m) o[i & 1][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < NS; ++k) {
+        if (!used(k)) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float4 a = *(const float4*)(lds_v[st] + (16 * k + 4 * grp + r) * D * 4 + 16 * col + 256 * i);
+          o[i & 1][0] = mma_f32(a.x, sv[k][r], o[i & 1][0]);
+          o[i & 1][1] = mma_f32(a.y, sv[k][r], o[i & 1][1]);
+          o[i & 1][2] = mma_f32(a.z, sv[k][r], o[i & 1][2]);
+          o[i & 1][3] = mma_f32(a.w, sv[k][r], o[i & 1][3]);
         }
       }
+      if (i >= LATE) add(i - LATE);
     }
+    if (LATE) add(NV - 1);
   };
   static_assert(RUN == 4, "a lane's dims: one float4 per 64");
 
@@ -510,19 +524,20 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(DecodeParams p, F32
     find_pages(0);
     load_step();
     find_pages(1);
-    store_step(0, 0);
+    store_step(0, 0, std::true_type{});
     __syncthreads();
     auto step = [&](int t, auto tail) {
-      if (t + 1 < steps) {
+      constexpr bool TAIL = decltype(tail)::value;
+      if (!TAIL || t + 1 < steps) {
         load_step();  // step t + 1
         find_pages(t + 2);
       }
       compute(t, t & 1, tail);
-      if (t + 1 < steps) store_step(t + 1, (t + 1) & 1);  // the stage of step t - 1
+      if (!TAIL || t + 1 < steps) store_step(t + 1, (t + 1) & 1, tail);  // the stage of step t - 1
       __syncthreads();
     };
     int t = 0;
-    for (const int whole = min_end > 0 ? min_end / KT : 0; t < whole; ++t) step(t, std::false_type{});
+    for (const int whole = mask_from > 0 ? mask_from / KT - 1 : 0; t < whole; ++t) step(t, std::false_type{});
     for (; t < steps; ++t) step(t, std::true_type{});
   }
   const float L = rows4_sum(l_run);
@@ -560,10 +575,10 @@ int f32_attend_launch(const DecodeParams& dp, int head_dim, int grid, hipStream_
 
 // From how many of its 64-row blocks per CU on the shared-K/V kernel is the
 // faster one: a block of it is a long serial job (900 keys at head_dim 256:
-// 155 us), where the other kernel has four times the workgroups.  us, other ->
-// shared, 900 keys: head_dim 256, 113 blocks 96 -> 161, 225 192 -> 159, 450
-// 382 -> 268; head_dim 128, 114 53 -> 82, 226 105 -> 82, 450 212 -> 146;
-// head_dim 64, 228 46 -> 48, 452 86 -> 78, 900 185 -> 155.
+// 168 us), where the other kernel has four times the workgroups.  us, other ->
+// shared, 900 keys: head_dim 256, 113 blocks 107 -> 168, 225 210 -> 180, 450
+// 409 -> 303; head_dim 128, 114 60 -> 84, 226 114 -> 90, 450 227 -> 153;
+// head_dim 64, 228 52 -> 53, 452 95 -> 83, 900 205 -> 160.
 static double shared_from(int head_dim) { return head_dim == 64 ? 1.5 : 0.8; }
 
 int f32_prefill_launch(const DecodeParams& dp, const int32_t* tile_hdr, const int2* tiles, int max_tiles,

@@ -49,3 +49,65 @@ def test_non_finite_v_reaches_its_16_row_blocks_only(gpu, heads, at, value):
         assert torch.equal(rows[~met], ref[~met])
         first = at - (kv - new)
         assert not bool(rows[first:].isfinite().any())
+
+
+def _attention64(q, k, v, first, scale):
+    """[tokens, heads, dim] attention in 64 bits; query i sees the keys up to first + i (all: first None)."""
+    g = q.shape[1] // k.shape[1]
+    out = torch.empty(q.shape, dtype=torch.float64, device=q.device)
+    for h in range(q.shape[1]):
+        s = (q[:, h].double() @ k[:, h // g].double().t().contiguous()) * scale
+        if first is not None:
+            at = torch.arange(q.shape[0], device=q.device)[:, None] + first
+            s.masked_fill_(torch.arange(k.shape[0], device=q.device)[None] > at, float("-inf"))
+        out[:, h] = torch.softmax(s, -1) @ v[:, h // g].double()
+    return out
+
+
+@pytest.mark.parametrize("heads", HEADS)
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("kv,new", [(2048, 1024), (900, 900)])
+def test_no_further_from_64_bits_than_the_16_row_kernel(gpu, heads, causal, kv, new):
+    """The same queries in batches too small for the kernel run through
+    attend_f32_kernel, whose sums are quarters of the keys long; a row's error is
+    random, so over a million outputs the two 2-norms compare to well under 5 %."""
+    hq, hkv, d = heads
+    ps = 16
+    meta = custom_batch([kv], ps, 140, 3, new_lens=[new])
+    cache = random_cache(140, ps, hkv, d, 5, F32).to(gpu)
+    q = torch.randn(new, hq, d, generator=torch.Generator().manual_seed(6)).to(gpu)
+    rows = cache[torch.as_tensor(meta[2]).long().to(gpu)].transpose(0, 1).reshape(2, -1, hkv, d)[:, :kv]
+    ref = _attention64(q, rows[0], rows[1], kv - new if causal else None, d ** -0.5)
+    shared = _wrapper(gpu, heads, ps, meta, causal).run(q, cache)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    part = int(0.7 * cus * 64 / hq)  # query tokens of a batch below the line
+    split = torch.empty_like(shared)
+    for a in range(0, new, part):
+        b = min(new, a + part)
+        seen = kv - new + b if causal else kv
+        m = custom_batch([seen], ps, 140, 3, new_lens=[b - a])  # the same pages
+        split[a:b] = _wrapper(gpu, heads, ps, m, causal).run(q[a:b], cache)
+    err = [float((o.double() - ref).norm() / ref.norm()) for o in (shared, split)]
+    log(f"f32 prefill {heads} causal={causal} kv={kv}: error shared {err[0]:.3e}, 16-row {err[1]:.3e}")
+    assert err[0] <= 1.05 * err[1]
+
+
+@pytest.mark.parametrize("heads", HEADS)
+def test_large_v_overflows_no_sooner_than_its_mean(gpu, heads):
+    """Probabilities relative to the row's max sum to at most the number of keys, so V
+    of 2^127 / keys keeps every partial sum finite, also where later keys score higher."""
+    hq, hkv, d = heads
+    log(f"f32 prefill, large V {heads}")
+    ps, kv, new = 16, 1024, 1000
+    meta = custom_batch([kv], ps, 70, 3, new_lens=[new])
+    cache = random_cache(70, ps, hkv, d, 5, F32).to(gpu)
+    pages = torch.as_tensor(meta[2]).long().to(gpu)
+    cache[pages, 1] = 2.0 ** 127 / kv
+    unit = torch.nn.functional.normalize(torch.randn(hkv, d, generator=torch.Generator().manual_seed(8)), dim=-1).to(gpu)
+    # scores rise with the key's position: by 5 (in exp2's terms 7.2) from first to last
+    rise = torch.linspace(0, 5, kv, device=gpu).view(-1, ps, 1, 1)
+    cache[pages, 0] = rise * unit * d ** 0.5
+    q = unit.repeat_interleave(hq // hkv, 0).expand(new, -1, -1).contiguous()
+    out = _wrapper(gpu, heads, ps, meta, False).run(q, cache)
+    assert bool(out.isfinite().all())
+    assert float((out / (2.0 ** 127 / kv) - 1).abs().max()) < 1e-5
