@@ -241,6 +241,22 @@ __device__ __forceinline__ int block_sum_1024(int v, int* smem) {
   return t;
 }
 
+// The max of v and, in sum, the sum of sum (smem: 32 ints).
+__device__ __forceinline__ int block_max_sum_1024(int v, int& sum, int* smem) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  v = wave_max(v);
+  sum = wave_sum(sum);
+  if (lane == 0) {
+    smem[w] = v;
+    smem[16 + w] = sum;
+  }
+  __syncthreads();
+  const int t = wave_max(smem[lane & 15]);
+  sum = wave_sum(lane < 16 ? smem[16 + lane] : 0);
+  __syncthreads();
+  return t;
+}
+
 __device__ __forceinline__ int block_max_1024(int v, int* smem) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   v = wave_max(v);
