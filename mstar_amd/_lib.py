@@ -329,13 +329,13 @@ class PinnedUploader:
 
 
 class PinnedRing:
-    """Pinned host rows that a launch reads by itself (``mi_*_plan_pinned``).
+    """Pinned host rows that a launch reads by itself (``mi_*_plan_pinned``), for one stream.
 
     ``SLOTS`` rows of ``VALUES`` int32 each are used in turn; an event recorded
     behind the launch guards a row until its next use, so a caller waits only
-    for the launch ``SLOTS`` calls ago.  Rows are never freed while a launch may
-    read them: use the per-device instance from :func:`pinned_ring`, which lives
-    for the process.
+    for the launch that was ``SLOTS`` calls ago on its own stream.  Rows are
+    never freed while a launch may read them: use the instances from
+    :func:`pinned_ring`, which live for the process.
     """
 
     SLOTS, VALUES = 8, 16384
@@ -352,7 +352,7 @@ class PinnedRing:
     def launch(self, parts, stream: int, fn) -> None:
         """Write ``parts`` (CPU tensors) one after the other and call ``fn(address)``, which launches on ``stream``."""
         _, record, sync = _events_api()
-        with self._lock:
+        with self._lock:  # held across the wait: the others here are on this stream, behind the same launch
             i = self._next
             self._next = (i + 1) % self.SLOTS
             ev = self._events[i]
@@ -370,17 +370,21 @@ class PinnedRing:
                 raise RuntimeError(f"hipEventRecord failed with HIP error {rc}")
 
 
+MAX_PINNED_RINGS = 64  # 512 KB of pinned memory each
 _rings: dict = {}
 
 
-def pinned_ring(device: torch.device) -> PinnedRing:
-    """The process-wide :class:`PinnedRing` of ``device``."""
-    r = _rings.get(device)
+def pinned_ring(device: torch.device, stream: int) -> PinnedRing:
+    """The process-wide :class:`PinnedRing` of ``stream`` on ``device``: a plan waits for none of
+    another stream's work.  Streams beyond the first ``MAX_PINNED_RINGS`` share one per device."""
+    r = _rings.get((device, stream))
     if r is None:
         with _uploaders_lock:
-            r = _rings.get(device)
+            if (device, stream) not in _rings and len(_rings) >= MAX_PINNED_RINGS:
+                stream = None
+            r = _rings.get((device, stream))
             if r is None:
-                r = _rings[device] = PinnedRing(device)
+                r = _rings[device, stream] = PinnedRing(device)
     return r
 
 

@@ -356,7 +356,7 @@ class PagedDecodeWrapper(_FusedRopeAppend):
                            "mi_decode_plan_host")
             elif pinned:
                 n_idx = paged_kv_indices.shape[0]
-                _lib.pinned_ring(dev).launch(
+                _lib.pinned_ring(dev, args[-1]).launch(
                     (paged_kv_indptr, paged_kv_last_page_len, paged_kv_indices), args[-1],
                     lambda at: _lib.check(_lib.lib().mi_decode_plan_pinned(at, n_idx, *args), "mi_decode_plan_pinned"))
             else:
@@ -563,7 +563,7 @@ class PagedPrefillWrapper(_FusedRopeAppend):
                        "mi_prefill_plan_host")
         elif pinned:
             n_idx = paged_kv_indices.shape[0]
-            _lib.pinned_ring(dev).launch(
+            _lib.pinned_ring(dev, args[-1]).launch(
                 (qo_indptr, paged_kv_indptr, paged_kv_last_page_len, paged_kv_indices), args[-1],
                 lambda at: _lib.check(_lib.lib().mi_prefill_plan_pinned(at, n_idx, *args), "mi_prefill_plan_pinned"))
         else:
