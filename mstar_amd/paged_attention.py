@@ -247,7 +247,35 @@ class _FusedRopeAppend:
                            k_scale, v_scale, keep_k, llama31)
 
 
-class PagedDecodeWrapper(_FusedRopeAppend):
+class _PlanArrays:
+    """The device arrays of a wrapper's plan, and the streams that read them.
+
+    They come from the planning stream's memory.  Where another stream reads
+    them (a run or append in an order the caller has made), the allocator is
+    told, so that they are not handed out again before that work is done, also
+    if the wrapper is dropped or planned anew in the meantime.  (The workspace
+    is the caller's; a plan rewrites it, so it has to be ordered behind the runs
+    of the last one.)  Static graph-mode buffers live as long as the wrapper."""
+
+    _plan_arrays: tuple = ()
+    _read_on: set = frozenset()
+
+    def _planned_on(self, stream: int, arrays) -> None:
+        self._plan_arrays = () if self.use_cuda_graph else arrays
+        self._read_on = {stream}
+
+    def _read_on_current(self) -> int:
+        """The current stream, known to the allocator as a reader of the plan."""
+        stream = _lib.stream_ptr(self.device)
+        if self._plan_arrays and stream not in self._read_on and not torch.cuda.is_current_stream_capturing():
+            here = torch.cuda.current_stream(self.device)
+            for t in self._plan_arrays:
+                t.record_stream(here)
+            self._read_on.add(stream)
+        return stream
+
+
+class PagedDecodeWrapper(_FusedRopeAppend, _PlanArrays):
     """Batched paged decode attention (``flashinfer_utils.py:291-484``)."""
 
     def __init__(
@@ -278,7 +306,6 @@ class PagedDecodeWrapper(_FusedRopeAppend):
         self.dtype = None
         self._workspace = workspace_buffer
         self._staging = _Staging()
-        self._indptr = self._retired = None
         self._n_req = 0
         if use_cuda_graph:
             assert batch_size is not None, "batch_size required for CUDA graph mode"
@@ -361,10 +388,10 @@ class PagedDecodeWrapper(_FusedRopeAppend):
                     lambda at: _lib.check(_lib.lib().mi_decode_plan_pinned(at, n_idx, *args), "mi_decode_plan_pinned"))
             else:
                 _lib.check(_lib.lib().mi_decode_plan(None, *args), "mi_decode_plan")
-        self._retired = self._indptr  # a run() of the previous plan may still read its arrays on another stream
         self._indptr, self._indices, self._last = indptr, indices, last
         self._n_req = n_req
         self.dtype = dtype
+        self._planned_on(args[-1], (indptr, indices, last, self.kv_cache_locations))
 
     def _adopt_plan(self, kv_indptr: torch.Tensor, kv_indices: torch.Tensor, last: torch.Tensor,
                     kv_cache_locations: torch.Tensor, dtype: torch.dtype) -> None:
@@ -386,6 +413,7 @@ class PagedDecodeWrapper(_FusedRopeAppend):
         self._indptr, self._indices, self._last = kv_indptr, kv_indices, last
         self._n_req = n_req
         self.dtype = dtype
+        self._planned_on(_lib.stream_ptr(self.device), (kv_indptr, kv_indices, last, self.kv_cache_locations))
 
     # --------------------------------------------------------------- run
     def run(self, q: torch.Tensor, kv_cache_layer: torch.Tensor, k_scale: torch.Tensor | None = None,
@@ -408,13 +436,14 @@ class PagedDecodeWrapper(_FusedRopeAppend):
         qs = _q_strides(q, "q")
         os_ = _q_strides(out, "out")
         batch = n
+        stream = self._read_on_current()
         _lib.check(
             _lib.lib().mi_decode_run(
                 q.data_ptr(), _lib.TORCH_TO_MI[q.dtype], qs[0], qs[1], desc, None, self._indptr.data_ptr(),
                 self._indices.data_ptr(), self._last.data_ptr(), batch, self.num_qo_heads, 0,
                 1.0 / math.sqrt(self.head_dim), self._workspace.data_ptr(),
                 self._workspace.numel() * self._workspace.element_size(), out.data_ptr(), os_[0], os_[1],
-                _lib.stream_ptr(q.device),
+                stream,
             ),
             "mi_decode_run",
         )
@@ -427,11 +456,12 @@ class PagedDecodeWrapper(_FusedRopeAppend):
 
     def _append_target(self):
         """(page ids, slot ids pointer, index stride, tokens, device token count) of this step's append."""
+        self._read_on_current()
         loc = self.kv_cache_locations
         return loc, loc.data_ptr() + 8, 2, self._n_req, None
 
 
-class PagedPrefillWrapper(_FusedRopeAppend):
+class PagedPrefillWrapper(_FusedRopeAppend, _PlanArrays):
     """Batched ragged paged prefill attention (``flashinfer_utils.py:70-288``)."""
 
     def __init__(
@@ -465,7 +495,6 @@ class PagedPrefillWrapper(_FusedRopeAppend):
         self.causal = True
         self._workspace = workspace_buffer
         self._staging = _Staging()
-        self._indptr = self._retired = None
         # Side stream of run(): made here so that a run() under graph capture
         # only records the fork/join on it (creating a stream is not capturable).
         self._side = torch.cuda.Stream(device=self.device)
@@ -568,9 +597,9 @@ class PagedPrefillWrapper(_FusedRopeAppend):
                 lambda at: _lib.check(_lib.lib().mi_prefill_plan_pinned(at, n_idx, *args), "mi_prefill_plan_pinned"))
         else:
             _lib.check(_lib.lib().mi_prefill_plan(*args), "mi_prefill_plan")
-        self._retired = self._indptr  # a run() of the previous plan may still read its arrays on another stream
         self._qo, self._indptr, self._indices, self._last = qo, indptr, indices, last
         self._n_req = n_req
+        self._planned_on(args[-1], (qo, indptr, indices, last, self.token_to_page, self.token_to_cache))
         self._serial = n_req <= _SERIAL_REQUESTS and (
             not self.use_cuda_graph or self.max_total_tokens * self.num_qo_heads <= _SERIAL_GRAPH_ROWS)
         self._plan_batch = batch
@@ -617,6 +646,7 @@ class PagedPrefillWrapper(_FusedRopeAppend):
         # of both, the HBM-bound decode runs on a side stream, so that it overlaps
         # the compute-bound tiles.
         main = torch.cuda.current_stream(q.device)
+        self._read_on_current()
         if self._run_tiles and self._run_short and self._serial:
             args[-1] = main.cuda_stream
             _lib.check(_lib.lib().mi_prefill_run(*args), "mi_prefill_run")
@@ -641,6 +671,7 @@ class PagedPrefillWrapper(_FusedRopeAppend):
 
     def _append_target(self):
         """(page ids, slot ids pointer, index stride, tokens, device token count) of this step's append."""
+        self._read_on_current()
         n_dev = self._qo.data_ptr() + 4 * self._n_req  # qo_indptr[n_req]: real count on the device
         return self.token_to_page, self.token_to_cache.data_ptr(), 1, self._total_tokens, n_dev
 

@@ -23,7 +23,7 @@ def _busy(gpu, seconds):
     torch.cuda._sleep(int(per * seconds / took))
     ev = torch.cuda.Event()
     ev.record()
-    return ev
+    return ev  # of the sleep: what is queued behind it has not begun before
 
 
 def test_a_pinned_plan_waits_for_no_other_stream(gpu):
@@ -56,3 +56,37 @@ def test_streams_beyond_the_last_ring_share_one(gpu, monkeypatch):
     rings = [_lib.pinned_ring(gpu, s) for s in (11, 12, 13, 14, 11, 13)]
     assert rings[0] is rings[4] and rings[0] is not rings[1]
     assert rings[2] is rings[3] is rings[5] and rings[2] not in rings[:2]
+
+
+@pytest.mark.parametrize("kind", ["decode", "prefill"])
+@pytest.mark.parametrize("pages", [40, 2000])  # indices in the launch argument; in pinned memory
+@pytest.mark.parametrize("part", ["run", "append"])
+def test_plan_arrays_outlive_a_reader_on_another_stream(gpu, kind, pages, part):
+    """Planned on one stream and read on another that is busy, then dropped: the plan's memory
+    is not handed out again while the reader is queued."""
+    log(f"{kind} plan of {pages} pages, {part} on another stream")
+    hq, hkv, d, ps = 8, 2, 128, 16
+    new = [1] if kind == "decode" else [60]
+    meta = [torch.as_tensor(x) for x in custom_batch([16 * pages], ps, pages, 3, new_lens=new)]
+    cache = torch.zeros(pages, 2, ps, hkv, d, dtype=torch.bfloat16, device=gpu)
+    q, k = (torch.zeros(new[0], h, d, dtype=torch.bfloat16, device=gpu) for h in (hq, hkv))
+    ws, out = workspace(gpu), torch.empty_like(q)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    cls = FlashInferDecodeWrapper if kind == "decode" else FlashInferPrefillWrapper
+    w = cls(ws, hq, hkv, d, ps, device=gpu)
+    w.plan(*meta[kind == "decode":])
+    mine = [(w._indices.data_ptr(), 4 * pages)] if part == "run" else [
+        (t.data_ptr(), t.numel() * 8) for t in ([w.kv_cache_locations] if kind == "decode" else [w.token_to_page])]
+    other = torch.cuda.Stream(gpu)
+    other.wait_stream(torch.cuda.current_stream(gpu))
+    with torch.cuda.stream(other):
+        done = _busy(gpu, 0.3)
+        w.run(q, cache, out=out) if part == "run" else w.set_kv_cache(cache, k, k)
+    del w
+    taken = [torch.empty(n // 4, dtype=torch.int32, device=gpu) for n in (mine[0][1], 4 * pages + 12, 16, 480)
+             for _ in range(40)]
+    overlap = [t for t in taken for a, n in mine if t.data_ptr() < a + n and a < t.data_ptr() + 4 * t.numel()]
+    assert not done.query(), "the reader is no longer queued: nothing was tested"
+    assert not overlap
+    torch.cuda.synchronize()
