@@ -3,6 +3,7 @@
 import pytest
 import torch
 
+import test_gpu_prefill_split as split
 from gpu_helpers import custom_batch, log, random_cache
 from mstar_amd import _lib
 from mstar_amd.paged_attention import FlashInferPrefillWrapper
@@ -80,3 +81,75 @@ def test_runs_that_state_another_workspace_size(gpu, heads, fp8):
             assert torch.equal(out, whole), (planned, ran, serial)
         small, _ = go(few, few, serial)
         assert torch.equal(go(few, roomy, serial)[0], small)
+
+
+@pytest.mark.parametrize("heads,ps,kv_lens,new", [
+    ((6, 3, 128), 16, [2500, 300], [150, 20]),    # 3, 6, 10 kv-heads: (piece, head) pairs in turn
+    ((24, 6, 64), 16, [2000], [90]),
+    ((10, 10, 256), 16, [900], [70]),
+    ((16, 16, 128), 32, [1700, 500], [60, 1]),    # 16 kv-heads: two a queue
+])
+def test_split_tiles_of_other_head_counts(gpu, heads, ps, kv_lens, new):
+    split.test_split_tiles_match_unsplit_and_fp32(gpu, heads, ps, kv_lens, new, True, torch.bfloat16, False)
+
+
+@pytest.mark.parametrize("heads", [(32, 4, 128), (32, 4, 64)])
+def test_whole_tiles_are_dealt(gpu, heads):
+    """With room for few partials, tiles of uneven requests are dealt uncut where that is
+    the better schedule; each tile's arithmetic, so every bit, is that of the local queues."""
+    hq, hkv, d = heads
+    log(f"whole tiles dealt {heads}")
+    ps, kv, new = 16, [2500, 9000, 1200, 5000], [500, 2000, 600, 1200]
+    meta = custom_batch(kv, ps, 1110, 3, new_lens=new)
+    cache = torch.randn(1110, 2, ps, hkv, d, device=gpu, dtype=torch.bfloat16)
+    q = torch.randn(sum(new), hq, d, device=gpu, dtype=torch.bfloat16)
+    full = _lib.lib().mi_prefill_workspace_bytes(len(kv), sum(new), hq, hkv, d)
+    outs = []
+    for room in (0, 2 * hkv):
+        ws = torch.empty(full - (768 - room) * 4 * 256 * d, dtype=torch.uint8, device=gpu)
+        w = FlashInferPrefillWrapper(ws, hq, hkv, d, ps, device=gpu)
+        w.plan(*(torch.as_tensor(x) for x in meta))
+        tiles, units, pieces, cut = _hdr(ws)[:4]
+        log(f"  room for {room} partials: tiles={tiles} pieces={pieces} split tiles={cut}")
+        assert cut == 0 and pieces == (tiles if room else 0) and units == tiles * hkv
+        outs.append(w.run(q, cache))
+        assert torch.equal(outs[-1], w.run(q, cache))
+    assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("at", [0, 700, 1090])
+def test_cut_plans_of_more_than_a_thread_per_tile(gpu, at):
+    """More than 1024 requests and tiles: two windows of each, and cut tiles on either side.
+
+    The bound is that of the split tests: with probabilities and outputs rounded to bf16,
+    |out - ref| <= 2^-8 (sum_i p_i |v_i| + 2 |ref|) + fp32 rounding."""
+    hq, hkv, d, ps = 8, 1, 256, 16
+    log(f"cut plan of 1102 requests, a long one at {at}")
+    kv, new = [20] * 1102, [20] * 1102
+    kv[at], new[at] = 24000, 320
+    kv[1101], new[1101] = 20000, 40
+    pool = int(sum(-(-n // ps) for n in kv))
+    meta = custom_batch(kv, ps, pool, 3, new_lens=new)
+    cache = torch.randn(pool, 2, ps, hkv, d, device=gpu, dtype=torch.bfloat16)
+    q = torch.randn(sum(new), hq, d, device=gpu, dtype=torch.bfloat16)
+    ws = torch.empty(512 << 20, dtype=torch.uint8, device=gpu)
+    w = FlashInferPrefillWrapper(ws, hq, hkv, d, ps, device=gpu)
+    w.plan_device(*(torch.as_tensor(x).to(gpu) for x in meta), total_tokens=sum(new))
+    tiles, _, pieces, cut = _hdr(ws)[:4]
+    log(f"  tiles={tiles} pieces={pieces} split tiles={cut}")
+    assert tiles > 1024 and pieces > tiles and cut > 0
+    out = w.run(q, cache)
+    qo, indptr, indices, _ = meta
+    worst = 0.0
+    for r in sorted({0, 1, 699, 700, 701, 1022, 1023, 1024, 1025, 1089, 1090, 1100, 1101}):
+        rows = cache[torch.as_tensor(indices[indptr[r]:indptr[r + 1]]).long().to(gpu)]
+        k, v = rows.transpose(0, 1).reshape(2, -1, d)[:, :kv[r]].double()
+        part = q[qo[r]:qo[r + 1]].double()
+        s = part @ k.t().contiguous() * d ** -0.5
+        seen = torch.arange(kv[r], device=gpu) <= torch.arange(kv[r] - new[r], kv[r], device=gpu)[:, None, None]
+        p = torch.softmax(s.masked_fill(~seen, float("-inf")), -1)
+        ref, mag = p @ v, p @ v.abs()
+        bound = 2.0 ** -8 * (mag + 2 * ref.abs()) + 1e-4
+        worst = max(worst, float(((out[qo[r]:qo[r + 1]].double() - ref).abs() / bound).max()))
+    log(f"  error/bound={worst:.2f}")
+    assert worst <= 1.0
