@@ -258,21 +258,25 @@ class _PlanArrays:
     of the last one.)  Static graph-mode buffers live as long as the wrapper."""
 
     _plan_arrays: tuple = ()
-    _read_on: set = frozenset()
+    _plan_stream: int | None = None
+    _readers: set = frozenset()
 
-    def _planned_on(self, stream: int, arrays) -> None:
-        self._plan_arrays = () if self.use_cuda_graph else arrays
-        self._read_on = {stream}
+    def _planned_on(self, stream: int, *arrays) -> None:
+        self._plan_stream, self._plan_arrays, self._readers = stream, arrays, frozenset()
 
-    def _read_on_current(self) -> int:
+    def _reading_stream(self) -> int:
         """The current stream, known to the allocator as a reader of the plan."""
         stream = _lib.stream_ptr(self.device)
-        if self._plan_arrays and stream not in self._read_on and not torch.cuda.is_current_stream_capturing():
+        if stream != self._plan_stream and not self.use_cuda_graph:
+            self._read_on(stream)
+        return stream
+
+    def _read_on(self, stream: int) -> None:
+        if stream not in self._readers and not torch.cuda.is_current_stream_capturing():
             here = torch.cuda.current_stream(self.device)
             for t in self._plan_arrays:
                 t.record_stream(here)
-            self._read_on.add(stream)
-        return stream
+            self._readers |= {stream}
 
 
 class PagedDecodeWrapper(_FusedRopeAppend, _PlanArrays):
@@ -391,7 +395,7 @@ class PagedDecodeWrapper(_FusedRopeAppend, _PlanArrays):
         self._indptr, self._indices, self._last = indptr, indices, last
         self._n_req = n_req
         self.dtype = dtype
-        self._planned_on(args[-1], (indptr, indices, last, self.kv_cache_locations))
+        self._planned_on(args[-1], indptr, indices, last, self.kv_cache_locations)
 
     def _adopt_plan(self, kv_indptr: torch.Tensor, kv_indices: torch.Tensor, last: torch.Tensor,
                     kv_cache_locations: torch.Tensor, dtype: torch.dtype) -> None:
@@ -413,7 +417,7 @@ class PagedDecodeWrapper(_FusedRopeAppend, _PlanArrays):
         self._indptr, self._indices, self._last = kv_indptr, kv_indices, last
         self._n_req = n_req
         self.dtype = dtype
-        self._planned_on(_lib.stream_ptr(self.device), (kv_indptr, kv_indices, last, self.kv_cache_locations))
+        self._planned_on(_lib.stream_ptr(self.device), kv_indptr, kv_indices, last, self.kv_cache_locations)
 
     # --------------------------------------------------------------- run
     def run(self, q: torch.Tensor, kv_cache_layer: torch.Tensor, k_scale: torch.Tensor | None = None,
@@ -436,7 +440,7 @@ class PagedDecodeWrapper(_FusedRopeAppend, _PlanArrays):
         qs = _q_strides(q, "q")
         os_ = _q_strides(out, "out")
         batch = n
-        stream = self._read_on_current()
+        stream = self._reading_stream()
         _lib.check(
             _lib.lib().mi_decode_run(
                 q.data_ptr(), _lib.TORCH_TO_MI[q.dtype], qs[0], qs[1], desc, None, self._indptr.data_ptr(),
@@ -456,7 +460,7 @@ class PagedDecodeWrapper(_FusedRopeAppend, _PlanArrays):
 
     def _append_target(self):
         """(page ids, slot ids pointer, index stride, tokens, device token count) of this step's append."""
-        self._read_on_current()
+        self._reading_stream()
         loc = self.kv_cache_locations
         return loc, loc.data_ptr() + 8, 2, self._n_req, None
 
@@ -599,7 +603,7 @@ class PagedPrefillWrapper(_FusedRopeAppend, _PlanArrays):
             _lib.check(_lib.lib().mi_prefill_plan(*args), "mi_prefill_plan")
         self._qo, self._indptr, self._indices, self._last = qo, indptr, indices, last
         self._n_req = n_req
-        self._planned_on(args[-1], (qo, indptr, indices, last, self.token_to_page, self.token_to_cache))
+        self._planned_on(args[-1], qo, indptr, indices, last, self.token_to_page, self.token_to_cache)
         self._serial = n_req <= _SERIAL_REQUESTS and (
             not self.use_cuda_graph or self.max_total_tokens * self.num_qo_heads <= _SERIAL_GRAPH_ROWS)
         self._plan_batch = batch
@@ -645,21 +649,17 @@ class PagedPrefillWrapper(_FusedRopeAppend, _PlanArrays):
         # short-query requests write disjoint rows: where the batch can hold much
         # of both, the HBM-bound decode runs on a side stream, so that it overlaps
         # the compute-bound tiles.
-        main = torch.cuda.current_stream(q.device)
-        self._read_on_current()
+        args[-1] = self._reading_stream()
         if self._run_tiles and self._run_short and self._serial:
-            args[-1] = main.cuda_stream
             _lib.check(_lib.lib().mi_prefill_run(*args), "mi_prefill_run")
         elif self._run_tiles and self._run_short:
-            side = self._side
+            main, side = torch.cuda.current_stream(q.device), self._side
             side.wait_stream(main)
-            args[-1] = main.cuda_stream
             _lib.check(_lib.lib().mi_prefill_tiles(*args), "mi_prefill_tiles")
             args[-1] = side.cuda_stream
             _lib.check(_lib.lib().mi_prefill_short(*args), "mi_prefill_short")
             main.wait_stream(side)
         elif self._run_tiles or self._run_short:
-            args[-1] = main.cuda_stream
             fn = "mi_prefill_tiles" if self._run_tiles else "mi_prefill_short"
             _lib.check(getattr(_lib.lib(), fn)(*args), fn)
         return out
@@ -671,7 +671,7 @@ class PagedPrefillWrapper(_FusedRopeAppend, _PlanArrays):
 
     def _append_target(self):
         """(page ids, slot ids pointer, index stride, tokens, device token count) of this step's append."""
-        self._read_on_current()
+        self._reading_stream()
         n_dev = self._qo.data_ptr() + 4 * self._n_req  # qo_indptr[n_req]: real count on the device
         return self.token_to_page, self.token_to_cache.data_ptr(), 1, self._total_tokens, n_dev
 
