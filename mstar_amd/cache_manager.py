@@ -467,10 +467,11 @@ class BatchedCacheManager:
         """Position ids for ``apply_rope`` (``cache_manager.py:426-520``).
 
         Without ``pos_ids``, request r contributes ``position_id_start[r] ..
-        + seq_lens[r] - 1``; the list is expanded on the GPU from one small
-        upload (cumulative lengths + starts) instead of a Python list of every
-        token.  In CUDA-graph mode an existing ``pos_ids`` buffer is rewritten
-        in place so captured launches keep their address.
+        + seq_lens[r] - 1``; the list is expanded on the GPU from the cumulative
+        lengths and starts (in the launch argument, or one small upload) instead
+        of a Python list of every token.  In CUDA-graph mode an existing
+        ``pos_ids`` buffer is rewritten in place so captured launches keep their
+        address.
         """
         nv = self.enable_nvtx
         with trace_range(nv, "cache.plan_rope"):
@@ -502,7 +503,7 @@ class BatchedCacheManager:
             else:
                 out = torch.empty(n, dtype=torch.long, device=self.device)
             if n:
-                # the positions are expanded on the device from one small upload
+                # the positions are expanded on the device
                 with trace_range(nv, "cache.plan_rope.copy_pos_ids"):
                     self._expand_positions(meta, b, out, n)
             ps.pos_ids = out

@@ -566,7 +566,7 @@ __global__ __launch_bounds__(1024) void prefill_plan_host_kernel(PfPlanArgs a, P
 // device copies) took the host 65 us a plan: 6 chunks and 17 decodes of up to
 // 5.7k tokens, a layer launched eagerly, 205 -> 139 us a pass; 4 chunks over up
 // to 8k cached tokens with an fp8 cache, bound by their tiles, 322 -> 317.  This kernel
-// 14 us on the former (bus reads in a chain of two).
+// 12.4 us on the former (bus reads in a chain of two).
 struct PfPinned {
   const int32_t* src;  // [qo_indptr | kv_indptr | last_page_len | kv_indices]
   int32_t num_indices, copy_blocks;

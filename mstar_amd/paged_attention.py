@@ -14,8 +14,9 @@ Differences from the reference, all deliberate:
 
 * No FlashInfer: planning runs on the GPU (``mi_decode_plan`` /
   ``mi_prefill_plan``) and never reads device memory back on the host.
-  ``plan()`` accepts CPU or device index tensors; CPU tensors go through one
-  pinned, asynchronous host->device copy.
+  ``plan()`` accepts CPU or device index tensors; CPU tensors travel in the plan
+  launch's argument, are read by it from pinned memory, or, large ones, go
+  through one pinned, asynchronous host->device copy.
 * ``set_kv_cache`` writes K and V in one kernel and, in CUDA-graph mode, skips
   the padding tokens beyond the planned count (the reference maps them to
   page 0 slot 0, ``flashinfer_utils.py:251-253``).
@@ -50,8 +51,11 @@ _MAX_GROUP = 16  # q heads per kv head handled by one MFMA tile
 # tokens 193 -> 176, two chunks and 14 decodes 239 -> 237; 8 chunks and 120
 # decodes 601 -> 635, so those fork).  A captured graph has no host in it, but
 # launches both parts whatever it is replayed on: in turn only where the tiles
-# are few (two 50-token suffixes, 8 layers: 247 -> 221; a 512-token chunk and 3
-# decodes 55 -> 58).
+# are few.  Up to _SERIAL_GRAPH_ROWS (token, q-head) rows in turn was 4-32 %
+# faster at head_dim 128 and -3 to 18 % at 256 (us a layer, forked -> in turn: two
+# 50-token suffixes at 8 q / 1 kv / 256 31.2 -> 25.5; 8192 rows with 14 decodes
+# 84.7 -> 78.4); at 12288 and 16384 rows 128 still gained 4-20 %, 256 lost up to 9 %
+# (a 2045-token chunk and 3 decodes 84.9 -> 92.7).
 _SERIAL_REQUESTS, _SERIAL_GRAPH_ROWS = 16, 8192
 
 
