@@ -48,6 +48,7 @@ struct F32Tiles {
   const int32_t* hdr;  // [0]: tiles listed by the prefill plan
   const int2* tiles;   // (request, first row)
   int32_t tile_rows;
+  int32_t from = 0, to = 0x7fffffff;  // the launch acts if the plan has from <= tiles < to
 };
 
 template <int D>
@@ -94,7 +95,8 @@ __global__ __launch_bounds__(256) void attend_f32_kernel(DecodeParams p, F32Tile
     const int j = x % bpt, rest = x / bpt;
     h = uniform(rest % nkv);
     const int t = rest / nkv;
-    if (t >= pt.hdr[0]) return;  // uniform
+    const int planned = pt.hdr[0];
+    if (t >= planned || planned >= pt.to) return;  // uniform
     const int2 tile = pt.tiles[t];
     b = uniform(tile.x);
     row0 = uniform(tile.y + kRows * j);
@@ -360,7 +362,8 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(DecodeParams p, F32
   const int x = (int)blockIdx.x;
   const int j = x % bpt, rest = x / bpt, t_idx = rest / nkv;
   const int h = uniform(rest - t_idx * nkv);
-  if (t_idx >= pt.hdr[0]) return;  // uniform
+  const int planned = pt.hdr[0];
+  if (t_idx >= planned || planned < pt.from) return;  // uniform
   const int2 tile = pt.tiles[t_idx];
   const int b = uniform(tile.x), row_wg = uniform(tile.y + 64 * j);
   const int page_base = p.kv_indptr[b];
@@ -574,31 +577,60 @@ int f32_attend_launch(const DecodeParams& dp, int head_dim, int grid, hipStream_
 }
 
 // From how many of its 64-row blocks per CU on the shared-K/V kernel is the
-// faster one: a block of it is a long serial job (900 keys at head_dim 256:
-// 168 us), where the other kernel has four times the workgroups.  us, other ->
-// shared, 900 keys: head_dim 256, 113 blocks 107 -> 168, 225 210 -> 180, 450
-// 409 -> 303; head_dim 128, 114 60 -> 84, 226 114 -> 90, 450 227 -> 153;
-// head_dim 64, 228 52 -> 53, 452 95 -> 83, 900 205 -> 160.
-static double shared_from(int head_dim) { return head_dim == 64 ? 1.5 : 0.8; }
+// faster one: a block of it is a long serial job and a CU runs two at a time, so
+// its time goes in steps (900 keys at head_dim 256: up to 1 block a CU 168 us, up
+// to 2 278), where the other kernel has four times the workgroups and cuts each
+// block's keys in four.  Under a causal mask the longest blocks set the step, so
+// the line lies higher; where the caller's graph forks the short-query part onto
+// another stream, that launch takes CUs in between and it lies higher still.
+// us, other -> shared, 900 keys, at 1.0 / 1.25 / 1.6 / 1.8 / 2.2 / 2.5 / 4 blocks a CU:
+//   head_dim 256  239 -> 272, 287 -> 276, 336 -> 278, 383 -> 280, 433 -> 444, 522 -> 464, 807 -> 676
+//     causal      149 -> 231, 163 -> 232, 218 -> 233, 248 -> 233, 300 -> 234, 322 -> 288, 505 -> 433
+//   head_dim 128  130 -> 136, 156 -> 137, 187 -> 138, 213 -> 140, 261 -> 208, 287 -> 208, 466 -> 330
+//     causal       85 -> 119,  92 -> 120, 124 -> 124, 145 -> 125, 173 -> 131, 185 -> 145, 296 -> 223
+//   head_dim 64    56 ->  74,  65 ->  75,  78 ->  76,  90 ->  77, 110 -> 115, 123 -> 115, 198 -> 180
+//     causal       50 ->  68,  53 ->  69,  55 ->  70,  65 ->  71,  78 ->  72,  79 ->  72, 126 -> 106
+// and 1800 keys at 1.25 and 1.6, head_dim 256: 506 -> 532, 593 -> 535.
+struct SharedFrom {
+  double plain, causal, forked, forked_causal;
+};
+static SharedFrom shared_from(int head_dim) {
+  if (head_dim == 64) return {2.3, 2.5, 4.0, 4.0};
+  if (head_dim == 128) return {1.4, 1.7, 1.8, 2.0};
+  return {1.6, 1.8, 1.6, 2.2};
+}
 
+// `rows` are exact in a plain call.  A captured one is replayed over plans of
+// fewer rows, so where the most rows would take the shared kernel it records
+// both, and the plan's tiles say which of them acts; the other exits at once (4
+// us).  A graph of up to 4096 tokens at 8 q / 1 kv / 256 over one request of 900:
+// 104 us a layer, 220 with the kernel chosen by the most rows.
 int f32_prefill_launch(const DecodeParams& dp, const int32_t* tile_hdr, const int2* tiles, int max_tiles,
                        int tile_rows, int64_t rows, int head_dim, hipStream_t stream) {
   if (tile_rows <= 0 || tile_rows % 64) return MI_ERR_INVALID;
   const int64_t blocks = (int64_t)max_tiles * dp.num_kv_heads * (tile_rows / 64);
-  if ((double)rows / 64 * dp.num_kv_heads >= shared_from(head_dim) * device_cu_count() && blocks <= 0x7fffffff) {
-    const F32Tiles pt{tile_hdr, tiles, tile_rows};
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &status) != hipSuccess) (void)hipGetLastError();
+  const bool captured = status == hipStreamCaptureStatusActive;
+  const SharedFrom line = shared_from(head_dim);
+  const double from = device_cu_count() * (captured ? (dp.causal ? line.forked_causal : line.forked)
+                                                    : (dp.causal ? line.causal : line.plain));
+  F32Tiles other{tile_hdr, tiles, tile_rows};
+  if ((double)rows / 64 * dp.num_kv_heads >= from && blocks <= 0x7fffffff) {
+    F32Tiles pt{tile_hdr, tiles, tile_rows};
+    if (captured) pt.from = other.to = (int)(from * 64 / ((double)dp.num_kv_heads * tile_rows)) + 1;
     switch (head_dim) {
       case 64: hipLaunchKernelGGL((prefill_f32_kernel<64>), dim3((int)blocks), dim3(256), 0, stream, dp, pt); break;
       case 128: hipLaunchKernelGGL((prefill_f32_kernel<128>), dim3((int)blocks), dim3(256), 0, stream, dp, pt); break;
       case 256: hipLaunchKernelGGL((prefill_f32_kernel<256>), dim3((int)blocks), dim3(256), 0, stream, dp, pt); break;
       default: return MI_ERR_UNSUPPORTED;
     }
-    return MI_OK;
+    if (!captured) return MI_OK;
   }
   const int64_t grid = (int64_t)max_tiles * dp.num_kv_heads * (tile_rows / kRows);
   if (grid <= 0) return MI_OK;
   if (grid > 0x7fffffff) return MI_ERR_UNSUPPORTED;
-  return dispatch_f32<true>(dp, F32Tiles{tile_hdr, tiles, tile_rows}, head_dim, (int)grid, stream);
+  return dispatch_f32<true>(dp, other, head_dim, (int)grid, stream);
 }
 
 }  // namespace mi
