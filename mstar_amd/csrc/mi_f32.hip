@@ -583,21 +583,23 @@ int f32_attend_launch(const DecodeParams& dp, int head_dim, int grid, hipStream_
 // block's keys in four.  Under a causal mask the longest blocks set the step, so
 // the line lies higher; where the caller's graph forks the short-query part onto
 // another stream, that launch takes CUs in between and it lies higher still.
-// us, other -> shared, 900 keys, at 1.0 / 1.25 / 1.6 / 1.8 / 2.2 / 2.5 / 4 blocks a CU:
-//   head_dim 256  239 -> 272, 287 -> 276, 336 -> 278, 383 -> 280, 433 -> 444, 522 -> 464, 807 -> 676
-//     causal      149 -> 231, 163 -> 232, 218 -> 233, 248 -> 233, 300 -> 234, 322 -> 288, 505 -> 433
-//   head_dim 128  130 -> 136, 156 -> 137, 187 -> 138, 213 -> 140, 261 -> 208, 287 -> 208, 466 -> 330
-//     causal       85 -> 119,  92 -> 120, 124 -> 124, 145 -> 125, 173 -> 131, 185 -> 145, 296 -> 223
-//   head_dim 64    56 ->  74,  65 ->  75,  78 ->  76,  90 ->  77, 110 -> 115, 123 -> 115, 198 -> 180
-//     causal       50 ->  68,  53 ->  69,  55 ->  70,  65 ->  71,  78 ->  72,  79 ->  72, 126 -> 106
+// us, other -> shared, 900 keys, at 0.9 / 1.0 / 1.25 / 1.6 / 1.8 / 2.2 / 2.5 / 4 blocks a CU:
+//   head_dim 256  195 -> 168, 239 -> 272, 287 -> 276, 336 -> 278, 383 -> 280, 433 -> 444, 522 -> 464, 807 -> 676
+//     causal      143 -> 163, 149 -> 231, 163 -> 232, 218 -> 233, 248 -> 233, 300 -> 234, 322 -> 288, 505 -> 433
+//   head_dim 128  109 ->  85, 130 -> 136, 156 -> 137, 187 -> 138, 213 -> 140, 261 -> 208, 287 -> 208, 466 -> 330
+//     causal       83 ->  84,  85 -> 119,  92 -> 120, 124 -> 124, 145 -> 125, 173 -> 131, 185 -> 145, 296 -> 223
+//   head_dim 64    49 ->  48,  56 ->  74,  65 ->  75,  78 ->  76,  90 ->  77, 110 -> 115, 123 -> 115, 198 -> 180
+//     causal       44 ->  46,  50 ->  68,  53 ->  69,  55 ->  70,  65 ->  71,  78 ->  72,  79 ->  72, 126 -> 106
 // and 1800 keys at 1.25 and 1.6, head_dim 256: 506 -> 532, 593 -> 535.
+// Without a mask the end of a step pays as well: [low, low_end), below the first
+// (head_dim 64: the second) full step.
 struct SharedFrom {
-  double plain, causal, forked, forked_causal;
+  double low, low_end, plain, causal, forked, forked_causal;
 };
 static SharedFrom shared_from(int head_dim) {
-  if (head_dim == 64) return {2.3, 2.5, 4.0, 4.0};
-  if (head_dim == 128) return {1.4, 1.7, 1.8, 2.0};
-  return {1.6, 1.8, 1.6, 2.2};
+  if (head_dim == 64) return {1.6, 1.9, 2.3, 2.2, 4.0, 4.0};
+  if (head_dim == 128) return {0.8, 0.96, 1.4, 1.7, 1.8, 2.0};
+  return {0.8, 0.96, 1.6, 1.8, 1.6, 2.2};
 }
 
 // `rows` are exact in a plain call.  A captured one is replayed over plans of
@@ -613,10 +615,12 @@ int f32_prefill_launch(const DecodeParams& dp, const int32_t* tile_hdr, const in
   if (hipStreamIsCapturing(stream, &status) != hipSuccess) (void)hipGetLastError();
   const bool captured = status == hipStreamCaptureStatusActive;
   const SharedFrom line = shared_from(head_dim);
-  const double from = device_cu_count() * (captured ? (dp.causal ? line.forked_causal : line.forked)
-                                                    : (dp.causal ? line.causal : line.plain));
+  const double cus = device_cu_count(), have = (double)rows / 64 * dp.num_kv_heads;
+  const double from = cus * (captured ? (dp.causal ? line.forked_causal : line.forked)
+                                      : (dp.causal ? line.causal : line.plain));
+  const bool low = !captured && !dp.causal && have >= line.low * cus && have < line.low_end * cus;
   F32Tiles other{tile_hdr, tiles, tile_rows};
-  if ((double)rows / 64 * dp.num_kv_heads >= from && blocks <= 0x7fffffff) {
+  if ((have >= from || low) && blocks <= 0x7fffffff) {
     F32Tiles pt{tile_hdr, tiles, tile_rows};
     if (captured) pt.from = other.to = (int)(from * 64 / ((double)dp.num_kv_heads * tile_rows)) + 1;
     switch (head_dim) {

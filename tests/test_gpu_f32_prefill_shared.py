@@ -20,7 +20,7 @@ from test_gpu_prefill import _run_prefill
 
 pytestmark = pytest.mark.gpu
 
-LINE = {256: 1.8, 128: 1.7, 64: 2.5}  # with a causal mask, where it lies higher
+LINE = {256: 1.8, 128: 1.7, 64: 2.3}  # with and without a causal mask
 
 
 @pytest.mark.parametrize("causal", [True, False])

@@ -1,6 +1,6 @@
 """GPU: the fp32 prefill kernel that shares K and V, over values that show what its sums meet.
 
-The sizes lie above the line from which it takes a batch (1.4-2.5 blocks of 64
+The sizes lie above the line from which it takes a batch (1.4-2.3 blocks of 64
 rows per CU).
 """
 
